@@ -78,6 +78,24 @@ struct TileLds {
 static_assert(sizeof(TileLds<kByteLdsTP, kByteLdsCap, kByteLdsWG>) + kByteLds + 128 <= 160 * 1024,
               "byte backend's LDS form: tables plus tile state must fit one CU's LDS");
 
+// A workgroup's next tile of a level: its own index first, then one from the
+// queue of those past the grid.  A level with no more tiles than workgroups
+// touches no counter: atomics on one address run one after the other, some
+// 9 ns each, and with one per tile and one more per workgroup to find the
+// queue empty a small level spent 20 us on them.
+struct TileQueue {
+    u32* ctr;
+    u32 ntiles;
+    bool first;
+    __device__ __forceinline__ u32 next() {
+        if (first) {
+            first = false;
+            return blockIdx.x;
+        }
+        return ntiles > gridDim.x ? gridDim.x + atomicAdd(ctr, 1u) : ntiles;
+    }
+};
+
 // Process every tile of one level (tiles come from a.tile_ctr).
 template <class SL, int TP, int CAP, int WG>
 __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, const int mode,
@@ -86,8 +104,9 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const u32 tp = (a.tile_parents && a.tile_parents < (u32)TP) ? a.tile_parents : (u32)TP;
     const u32 ntiles = (a.n_in + tp - 1) / tp;
+    TileQueue q{a.tile_ctr, ntiles, true};
     for (;;) {
-        if (tid == 0) s.tile = atomicAdd(a.tile_ctr, 1u);
+        if (tid == 0) s.tile = q.next();
         __syncthreads();
         const u32 tile = s.tile;
         if (tile >= ntiles) break;
@@ -163,7 +182,7 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
                 if (t && uni && a.root_sums) atomicAdd(&a.root_sums[r0], t);
             }
         }
-        if (!uni && ps && a.root_sums) atomicAdd(&a.root_sums[s.root[tid]], (unsigned long long)ps);
+        if (!uni && a.root_sums) wave_run_add((u32)tid < np ? &a.root_sums[s.root[tid]] : nullptr, ps);
         __syncthreads();
     }
 }

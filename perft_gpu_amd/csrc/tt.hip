@@ -47,27 +47,6 @@ constexpr int kTTLeafWaves = 5;
 // is taken with one atomic.
 constexpr int kTTMixedWaves = 5;
 
-// Adds each lane's v to its *p with one global atomic per run of consecutive
-// lanes that hold the same address.  A level's children are written in their
-// parents' order, so the 64 items of an upsweep wave usually belong to two or
-// three parents; the run's head lane adds the run's total.  Every lane of the
-// wave must call it; a lane with p == nullptr adds nothing.
-__device__ __forceinline__ void wave_run_add(unsigned long long* p, unsigned long long v) {
-    const int lane = threadIdx.x & 63;
-    const unsigned long long a = reinterpret_cast<unsigned long long>(p);
-    const unsigned long long prev = __shfl_up(a, 1, 64);
-    const bool head = lane == 0 || prev != a;
-    const unsigned long long heads = __ballot(head);
-    const u32 rid = (u32)__popcll(heads & ((2ULL << lane) - 1));  // runs that start at or below this lane
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {  // suffix sums within each run
-        const unsigned long long ov = __shfl_down(v, d, 64);
-        const u32 orid = __shfl_down(rid, d, 64);
-        if (lane + d < 64 && orid == rid) v += ov;
-    }
-    if (head && p && v) atomicAdd(p, v);
-}
-
 __device__ __forceinline__ bool tt_probe(const uint4* tt, u64 mask, u64 k1, u64 k2, int depth, u64* val) {
     const uint4* bkt = tt + 2 * tt_bucket(k1, depth, mask);
 #pragma unroll
