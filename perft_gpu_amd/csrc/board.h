@@ -27,6 +27,8 @@ constexpr u64 kRanks2to7 = 0x00FFFFFFFFFFFF00ULL;
 constexpr u64 kRank1 = 0x00000000000000FFULL;
 constexpr u64 kRank3 = 0x0000000000FF0000ULL;
 constexpr u64 kRank5 = 0x000000FF00000000ULL;
+constexpr u64 kRank6 = 0x0000FF0000000000ULL;
+constexpr u64 kRank7 = 0x00FF000000000000ULL;
 constexpr u64 kRank8 = 0xFF00000000000000ULL;
 constexpr u64 kFileA = 0x0101010101010101ULL;
 constexpr u64 kFileH = 0x8080808080808080ULL;
@@ -146,6 +148,36 @@ PF_HD u64 shr(u64 x) {
     }
 #endif
     return x >> S;
+}
+
+// Ends a stage of a long computation on the GPU: the values named are
+// computed before it, others are computed (or read from memory) again after
+// it rather than kept in registers.
+PF_HD void pin(u64& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#endif
+}
+PF_HD void pin(u32& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#endif
+}
+// Whether x is not 0 in any lane of the wave (on the host: of this call).
+PF_HD bool any_lane(u64 x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __ballot(x != 0) != 0;
+#else
+    return x != 0;
+#endif
+}
+template <class... T>
+PF_HD void stage_end(T&... x) {
+    (pin(x), ...);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
 }
 
 // Kogge-Stone occluded fills: `g` generators, `p` propagator (empty squares).
@@ -273,6 +305,15 @@ PF_HD u64 diag_of(int s) {  // a1-h8 direction
 }
 PF_HD u64 anti_of(int s) {  // a8-h1 direction
     return shift_rows(0x0102040810204080ULL, (s & 56) + ((s & 7) << 3) - 56);
+}
+
+// Attacks along one line mask `m` (through s) of a slider on s: both rays by
+// obstruction difference, (o - 2s) ^ o for the squares above s and the same
+// on the bit-reversed board for those below.  `rocc` = reverse(occ).
+PF_HD u64 reverse(u64 x) { return __builtin_bitreverse64(x); }
+PF_HD u64 line_attack(u64 m, u64 occ, u64 rocc, u64 sb, u64 rsb) {
+    const u64 up = (occ & m) - (sb << 1), dn = (rocc & reverse(m)) - (rsb << 1);
+    return bitop3<0x28>(up, reverse(dn), m);  // (up ^ down) & m
 }
 
 }  // namespace pf

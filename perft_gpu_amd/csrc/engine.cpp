@@ -153,9 +153,9 @@ pf_status Engine::expand(int mode, const Board* in, const u32* in_root, u64 n_in
     a.total = next_total ? d_total : nullptr;
     a.tile_ctr = d_ctrl + 1;
     a.err = d_ctrl + 0;
-    // a level with fewer than 64 parents per workgroup of the wide launch is
+    // a level with few parents per workgroup of the wide launch is
     // latency-bound: it takes the small-level shape
-    const int small = n_in < (u64)grid[backend][mode] * 64 ? 1 : 0;
+    const int small = n_in < (u64)grid[backend][mode] * (mode == kLeaf ? kLeafSetsMinParents : 64) ? 1 : 0;
     int g = small ? grid_small[backend][mode] : grid[backend][mode];
     a.tile_parents = level_tile_parents(n_in, (u64)g, 256);
     const u64 tiles = (n_in + a.tile_parents - 1) / a.tile_parents;

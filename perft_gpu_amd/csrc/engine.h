@@ -45,7 +45,7 @@ struct Engine {
         int p_bpc = 0;        // persistent kernel workgroups per CU
         int tt_bpc = 0;       // TT write-level kernel workgroups per CU
         int single_pass = 0;  // table-free batches under PF_MODE_AUTO: 0 stream-ordered levels, 1 cooperative
-        int s_leaf = kStreamLeafDefault;    // stream-ordered leaf-level kernel form (stream.hip)
+        int s_leaf = kStreamLeafSets;       // stream-ordered leaf-level kernel form (stream.hip)
         int s_write = kStreamWriteDefault;  // stream-ordered write-level kernel form
         int tt_leaf_bpc = 0;  // TT leaf-level kernel workgroups per CU
         int tt_chunk_pct = 50;  // TT level driver: a chunk's next level may take this share of the free arena

@@ -36,6 +36,9 @@ PF_HD u32 level_tile_parents(u64 n, u64 grid, u32 tp_max) {
     return (u32)(t < 1 ? 1 : t > tp_max ? tp_max : t);
 }
 
+// A leaf level runs by sets (leaf.h) from this many parents per workgroup.
+constexpr u32 kLeafSetsMinParents = 32;
+
 enum ExpandMode : int { kLeaf = 0, kWrite = 1 };
 
 // Occupancy-derived grid size for the expand kernel (workgroups); small = 1
@@ -79,13 +82,13 @@ hipError_t launch_persistent(int backend, int variant, const DevTables& dt, cons
 // The same batch as one launch per level on stream s (levels sized and placed
 // on the device; no host round trip): the root count, then depth - 1 level
 // launches of grid[kWrite] / grid[kLeaf] workgroups of the level kernel's
-// form variant[kWrite] / variant[kLeaf] (stream.hip: tile shape * 3 + waves
-// per SIMD target; the byte backend has one form).
-constexpr int kStreamVariants = 6;
-constexpr int kStreamWriteVariants = 5;  // the write kernel has no five-wave 256 x 4096 form
+// form variant[kWrite] / variant[kLeaf].  Write levels have kStreamWriteVariants
+// forms (stream.hip: tile shape * 3 + waves per SIMD target), the leaf level
+// one, by sets; both have one more for the byte backend.
+constexpr int kStreamWriteVariants = 5;  // (there is no five-wave 256 x 4096 write form)
 constexpr int kStreamByteLds = 6;        // byte backend only: its tables staged in LDS (both modes)
-constexpr int kStreamLeafDefault = 5;   // 256 x 4096 tile, five waves per SIMD
-constexpr int kStreamWriteDefault = 3;  // 256 x 4096 tile, no waves target
+constexpr int kStreamLeafSets = 7;       // leaf level by sets (leaf.h); below kLeafSetsMinParents move by move
+constexpr int kStreamWriteDefault = 3;   // 256 x 4096 tile, no waves target
 int stream_grid(int backend, int mode, int variant, int n_cu);
 hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a, const int grid[2],
                          const int variant[2], hipStream_t s);

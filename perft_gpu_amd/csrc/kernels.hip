@@ -27,16 +27,24 @@
 namespace pf {
 
 
-// The host-driven level loop has both shapes: the wide one above for large
-// levels, and for small ones (few parents per workgroup, latency-bound) the
-// 256 x 8192 tile without a waves-per-SIMD target, which does not spill.
+// The host-driven level loop has two shapes: for write levels a wide one (V =
+// 2) on large levels, and for both modes, on small ones (few parents per
+// workgroup, latency-bound), the 256 x 8192 tile (V = 0).
 template <int B, int MODE, int V>
-__global__ __launch_bounds__(kWG)
-__attribute__((amdgpu_waves_per_eu(V == LevelV<B>::v ? LevelWaves<B, MODE>::v : 1)))
-void k_expand(const SliderTables* tabs, LevelArgs a) {
+__global__ __launch_bounds__(kWG) void k_expand(const SliderTables* tabs, LevelArgs a) {
     __shared__ TileLds<PCfg<B, V>::TP, PCfg<B, V>::CAP, kWG> s;
     const auto sl = SlOf<B>::make(tabs);
     expand_level(sl, a, MODE, s);
+}
+
+// The leaf level by sets (leaf.h), for levels of at least kLeafSetsMinParents
+// parents per workgroup.
+template <int B>
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(kLeafSetsWaves)))
+void k_expand_leaf(const SliderTables* tabs, LevelArgs a) {
+    __shared__ LeafLevelLds s;
+    const auto sl = SlOf<B>::make(tabs);
+    leaf_level(sl, a, s);
 }
 
 template <int B>
@@ -91,10 +99,15 @@ __global__ __launch_bounds__(kWG) void k_range_count(const Board* b, u32 n, unsi
 // All branch decisions between barriers read the same device words, so every
 // workgroup takes the same path and reaches every barrier.
 template <int B, int V>
-__global__ __launch_bounds__(kWG) void k_persistent(const SliderTables* tabs, PersistArgs p) {
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(kLeafSetsWaves)))
+void k_persistent(const SliderTables* tabs, PersistArgs p) {
     namespace cg = cooperative_groups;
     cg::grid_group grid = cg::this_grid();
-    __shared__ TileLds<PCfg<B, V>::TP, PCfg<B, V>::CAP, kWG> s;
+    __shared__ union {
+        TileLds<PCfg<B, V>::TP, PCfg<B, V>::CAP, kWG> tile;
+        LeafLevelLds sets;
+    } lds;
+    auto& s = lds.tile;
     const auto sl = SlOf<B>::make(tabs);
     PersistCtl* ctl = p.ctl;
 
@@ -127,7 +140,9 @@ __global__ __launch_bounds__(kWG) void k_persistent(const SliderTables* tabs, Pe
             a.out_cap = 0;
             a.root_sums = p.sums;
             a.total = nullptr;
-            expand_level(sl, a, kLeaf, s);
+            a.tile_parents = level_tile_parents(n, gridDim.x, 256);
+            if (a.tile_parents >= kLeafSetsMinParents) leaf_level(sl, a, lds.sets);
+            else expand_level(sl, a, kLeaf, s);
             break;
         }
         const u64 nn = __hip_atomic_load(&ctl->totals[L + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -157,7 +172,8 @@ __global__ __launch_bounds__(kWG) void k_persistent(const SliderTables* tabs, Pe
 template <int B, int MODE>
 static void* expand_fn(int small) {
     if (small) return reinterpret_cast<void*>(&k_expand<B, MODE, 0>);
-    return reinterpret_cast<void*>(&k_expand<B, MODE, LevelV<B>::v>);
+    if constexpr (MODE == kLeaf) return reinterpret_cast<void*>(&k_expand_leaf<B>);
+    else return reinterpret_cast<void*>(&k_expand<B, MODE, 2>);
 }
 
 static void* pick_expand(int backend, int mode, int small) {

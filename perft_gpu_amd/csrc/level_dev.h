@@ -6,6 +6,7 @@
 
 #include "backends_dev.h"
 #include "kernels.h"
+#include "leaf_dev.h"
 #include "wave.h"
 
 namespace pf {
@@ -187,6 +188,62 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
     }
 }
 
+// The leaf level by sets (leaf.h): 256 parents a tile, one per thread.  The
+// record pools hold ten records a parent and the move list 1,280 moves (a
+// tile of middlegame positions hands out some 820 records and 1,030 moves to
+// be counted in full, then 750 of which only the king's replies are), which
+// leaves room for three workgroups in a CU's LDS, as many as the kernel's 164
+// VGPRs allow.
+// Per-level kernels take it from kLeafSetsMinParents parents per workgroup: below,
+// a wave has too few parents for its long pass over each, and the leaf level
+// runs move by move.  16 roots at perft 4 (20 parents per workgroup): 60 us
+// move by move, 65 by sets; 32 roots (40): 86 against 83; 256 roots (320):
+// 283 against 179.
+constexpr int kLeafSetsWaves = 3;
+struct LeafLevelLds {
+    LeafLds<256, 640, 1280, kWG> t;
+    u32 root[256];
+    unsigned long long red[kWG / 64];
+    u32 tile;
+};
+
+// Process every tile of the leaf level (tiles come from a.tile_ctr).
+template <class SL>
+__device__ __forceinline__ void leaf_level(const SL& sl, const LevelArgs& a, LeafLevelLds& s) {
+    const u32 tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const u32 tp = (a.tile_parents && a.tile_parents < 256u) ? a.tile_parents : 256u;
+    const u32 ntiles = (a.n_in + tp - 1) / tp;
+    TileQueue q{a.tile_ctr, ntiles, true};
+    for (;;) {
+        if (tid == 0) s.tile = q.next();
+        __syncthreads();
+        const u32 tile = s.tile;
+        if (tile >= ntiles) break;
+        const u32 p0 = tile * tp;
+        const u32 np = min(tp, a.n_in - p0);
+        s.t.b[tid] = tid < np ? a.in[p0 + tid] : Board{};
+        s.root[tid] = tid < np ? a.in_root[p0 + tid] : 0u;
+        __syncthreads();
+        leaf_tile(sl, np, s.t);
+        const u32 ps = tid < np ? s.t.sum[tid] : 0u;
+        const u32 r0 = s.root[0];
+        if (__syncthreads_and(tid >= np || s.root[tid] == r0)) {
+            const unsigned long long v = wave_sum64((unsigned long long)ps);
+            if (lane == 0) s.red[wid] = v;
+            __syncthreads();
+            if (tid == 0) {
+                unsigned long long t = 0;
+#pragma unroll
+                for (int w = 0; w < kWG / 64; w++) t += s.red[w];
+                if (t) atomicAdd(&a.root_sums[r0], t);
+            }
+        } else {
+            wave_run_add(tid < np ? &a.root_sums[s.root[tid]] : nullptr, ps);
+        }
+        __syncthreads();
+    }
+}
+
 // Tile shapes of the persistent kernel that the tuner chooses between:
 // variant 0 = 256 parents x 8192-entry move window, 1 = 128 x 4096,
 // 2 = 256 x 4096.
@@ -196,25 +253,6 @@ struct PCfg {
     static constexpr int CAP = (V == 0) ? 8192 : 4096;
 };
 
-// Tile shape of the per-level kernels (k_expand, k_stream_level): 256 x 4096
-// (variant 2), whose smaller LDS footprint lets more workgroups share a CU
-// than the 256 x 8192 shape.
-template <int B>
-struct LevelV {
-    static constexpr int v = 2;
-};
-// Waves per SIMD the per-level kernels are built for (1 = no constraint).
-// The leaf kernel is built for five, so five workgroups share a CU; the magic
-// backends' fits 96 VGPRs as it is, Kogge-Stone's spills a few bytes per lane
-// (outside its make+count loop).  C2 leaves/s of the stream-ordered form,
-// 256 x 8192 at three per CU -> 256 x 4096 at four -> at five: plain 1.05e12
-// -> 1.18e12 -> 1.30e12, fancy 1.08e12 -> 1.20e12 -> 1.31e12 (their table
-// reads from L2 want the extra waves), Kogge-Stone 1.470e12 -> 1.479e12 ->
-// 1.500e12.  The write kernels would spill more and stay at four.
-template <int B, int MODE>
-struct LevelWaves {
-    static constexpr int v = (MODE == kLeaf) ? 5 : 1;
-};
 // Workgroups of one of these kernels that fit a CU (a kernel with dynamic LDS
 // has it enabled first).
 static inline int blocks_per_cu(void* f, int wg = kWG, size_t dyn = 0) {

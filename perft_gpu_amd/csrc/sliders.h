@@ -49,8 +49,16 @@ struct SliderTables {
 
 struct KSBackend {
     static constexpr bool kSetwise = true;
-    PF_HD u64 rook(int s, u64 occ) const { return rook_fill(bit(s), ~occ); }
-    PF_HD u64 bishop(int s, u64 occ) const { return bishop_fill(bit(s), ~occ); }
+    // One slider: two lines by obstruction difference, about 20 instructions
+    // each, where two occluded fills take 44.
+    PF_HD u64 rook(int s, u64 occ) const {
+        const u64 r = reverse(occ), sb = bit(s), rs = reverse(sb);
+        return line_attack(file_of(s), occ, r, sb, rs) | line_attack(rank_of(s), occ, r, sb, rs);
+    }
+    PF_HD u64 bishop(int s, u64 occ) const {
+        const u64 r = reverse(occ), sb = bit(s), rs = reverse(sb);
+        return line_attack(diag_of(s), occ, r, sb, rs) | line_attack(anti_of(s), occ, r, sb, rs);
+    }
     PF_HD u64 rook_multi(u64 set, u64 occ) const { return rook_fill(set, ~occ); }
     PF_HD u64 bishop_multi(u64 set, u64 occ) const { return bishop_fill(set, ~occ); }
 };

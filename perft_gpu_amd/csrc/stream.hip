@@ -8,22 +8,19 @@
 // Every workgroup of a level launch derives the same placement from words
 // the previous launch finished writing.
 //
-// The level kernel is built in kStreamVariants forms -- two tile shapes times
-// three waves-per-SIMD targets -- for the leaf mode and in the first five of
-// them for the write mode, and the autotuner picks the leaf and the write
-// form per backend (the reference fixes its launch shape at compile time,
-// perft_bb.h:327-329, switches.h:14-21).
+// The write kernel is built in kStreamWriteVariants forms -- two tile shapes
+// times three waves-per-SIMD targets, less the last -- of which the autotuner
+// picks one per backend (the reference fixes its launch shape at compile time,
+// perft_bb.h:327-329, switches.h:14-21).  The leaf level runs by sets (leaf.h).
 //
 // The write kernel's 256 x 4096 form built for five waves per SIMD (96
-// VGPRs, over 100 B of spills per lane) is not built: compiled from the
-// current make-move and count code with the current compiler, it gave counts
-// that differ from the oracle's on a perft 4 sample, and differently from run
-// to run.  Its other forms, the leaf kernel's five-wave forms, and the same
-// form built with only one of the two latest changes to that code (the
-// flag decoding of make_move, the branch-free diagonal masks) all match.  No
-// cause in the source was found: the LDS tile is fenced by barriers and every
-// spill slot lies inside the declared private segment.  The form was never a
-// tuned choice: the write level spills more than it gains at that target.
+// VGPRs, over 100 B of spills per lane) is not built: it gave counts that
+// differ from the oracle's on a perft 4 sample, and differently from run to
+// run, and no cause in the source was found.  The leaf level's kernels are
+// kept free of spills for the same reason: built for four waves per SIMD (128
+// VGPRs, 44 B of spills per lane) their sums differed from run to run as soon
+// as two workgroups shared a compute unit, while the three-wave build (164
+// VGPRs, no spills) of the same source is exact and as fast.
 #include <hip/hip_runtime.h>
 
 #include "level_dev.h"
@@ -60,9 +57,9 @@ __global__ __launch_bounds__(kWG) void k_stream_roots(const SliderTables* tabs, 
 // One level for one workgroup of the launch.  `make_sl` builds the slider
 // backend once the workgroup knows it has work (the byte backend's LDS form
 // copies its tables into LDS there).
-template <int MODE, int TP, int CAP, int WG, class MakeSl>
+template <int MODE, bool SETS, int TP, int CAP, int WG, class MakeSl>
 __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const PersistArgs& p, int L,
-                                             TileLds<TP, CAP, WG>& s) {
+                                             TileLds<TP, CAP, WG>& s, LeafLevelLds* sets) {
     PersistCtl* ctl = p.ctl;
     // an earlier level did not fit: nothing below it is counted (one read per
     // workgroup, so that the whole workgroup leaves together)
@@ -98,6 +95,12 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
         a.out_cap = 0;
         a.root_sums = p.sums;
         a.total = nullptr;
+        if constexpr (SETS) {
+            if (a.tile_parents >= kLeafSetsMinParents) {
+                leaf_level(sl, a, *sets);
+                return;
+            }
+        }
         expand_level(sl, a, kLeaf, s);
         return;
     }
@@ -118,12 +121,12 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
     expand_level(sl, a, kWrite, s);
 }
 
-template <int B, int MODE, int SH, int WV>
+template <int B, int SH, int WV>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(StreamWaves<WV>::v)))
-void k_stream_level(const SliderTables* tabs, PersistArgs p, int L) {
+void k_stream_write(const SliderTables* tabs, PersistArgs p, int L) {
     using Shape = PCfg<B, StreamShape<SH>::v>;
     __shared__ TileLds<Shape::TP, Shape::CAP, kWG> s;
-    stream_level<MODE>([&] { return SlOf<B>::make(tabs); }, p, L, s);
+    stream_level<kWrite, false>([&] { return SlOf<B>::make(tabs); }, p, L, s, nullptr);
 }
 
 // The byte backend's LDS form (level_dev.h): one 768-thread workgroup per CU,
@@ -132,36 +135,41 @@ template <int MODE>
 __global__ __launch_bounds__(kByteLdsWG) void k_stream_level_byte_lds(const SliderTables* tabs, PersistArgs p, int L) {
     extern __shared__ __align__(16) unsigned char dyn_lds[];
     __shared__ TileLds<kByteLdsTP, kByteLdsCap, kByteLdsWG> s;
-    stream_level<MODE>([&] { return stage_byte_tables(tabs, dyn_lds); }, p, L, s);
+    stream_level<MODE, false>([&] { return stage_byte_tables(tabs, dyn_lds); }, p, L, s, nullptr);
+}
+
+// The leaf level by sets; a level too small for it runs move by move.
+template <int B>
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(kLeafSetsWaves)))
+void k_stream_leaf(const SliderTables* tabs, PersistArgs p, int L) {
+    __shared__ union {
+        TileLds<256, 4096, kWG> tile;
+        LeafLevelLds sets;
+    } s;
+    stream_level<kLeaf, true>([&] { return SlOf<B>::make(tabs); }, p, L, s.tile, &s.sets);
 }
 
 // ---- launch plumbing --------------------------------------------------------
-template <int B, int MODE>
-static void* level_fn(int v) {
-    switch (v) {
-    case 0: return reinterpret_cast<void*>(&k_stream_level<B, MODE, 0, 0>);
-    case 1: return reinterpret_cast<void*>(&k_stream_level<B, MODE, 0, 1>);
-    case 2: return reinterpret_cast<void*>(&k_stream_level<B, MODE, 0, 2>);
-    case 3: return reinterpret_cast<void*>(&k_stream_level<B, MODE, 1, 0>);
-    case 4: return reinterpret_cast<void*>(&k_stream_level<B, MODE, 1, 1>);
-    default:
-        if constexpr (MODE == kWrite) return reinterpret_cast<void*>(&k_stream_level<B, MODE, 1, 1>);
-        else return reinterpret_cast<void*>(&k_stream_level<B, MODE, 1, 2>);
-    }
-}
 template <int B>
-static void* level_fn_mode(int mode, int v) {
-    return mode == kWrite ? level_fn<B, kWrite>(v) : level_fn<B, kLeaf>(v);
+static void* level_fn(int mode, int v) {
+    if (mode == kLeaf) return reinterpret_cast<void*>(&k_stream_leaf<B>);
+    switch (v) {
+    case 0: return reinterpret_cast<void*>(&k_stream_write<B, 0, 0>);
+    case 1: return reinterpret_cast<void*>(&k_stream_write<B, 0, 1>);
+    case 2: return reinterpret_cast<void*>(&k_stream_write<B, 0, 2>);
+    case 3: return reinterpret_cast<void*>(&k_stream_write<B, 1, 0>);
+    default: return reinterpret_cast<void*>(&k_stream_write<B, 1, 1>);
+    }
 }
 static void* pick_stream_level(int backend, int mode, int v) {
     if (backend == kByte && v == kStreamByteLds)
         return mode == kWrite ? reinterpret_cast<void*>(&k_stream_level_byte_lds<kWrite>)
                               : reinterpret_cast<void*>(&k_stream_level_byte_lds<kLeaf>);
     switch (backend) {
-    case kKS: return level_fn_mode<kKS>(mode, v);
-    case kPlain: return level_fn_mode<kPlain>(mode, v);
-    case kFancy: return level_fn_mode<kFancy>(mode, v);
-    default: return level_fn_mode<kByte>(mode, v);
+    case kKS: return level_fn<kKS>(mode, v);
+    case kPlain: return level_fn<kPlain>(mode, v);
+    case kFancy: return level_fn<kFancy>(mode, v);
+    default: return level_fn<kByte>(mode, v);
     }
 }
 static void* pick_stream_roots(int backend) {

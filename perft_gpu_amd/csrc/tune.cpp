@@ -31,8 +31,9 @@ void Engine::apply_tuning() {
         Tune& t = tune[b];
         if (t.p_variant < 0 || t.p_variant >= kPersistVariants) t.p_variant = 0;
         const bool lds_form_ok = b == kByte;
-        if (t.s_leaf < 0 || (t.s_leaf >= kStreamVariants && !(lds_form_ok && t.s_leaf == kStreamByteLds)))
-            t.s_leaf = kStreamLeafDefault;
+        // (files may name leaf forms 0 to 5, which ran every leaf move by move
+        // and are no longer built)
+        if (!(lds_form_ok && t.s_leaf == kStreamByteLds)) t.s_leaf = kStreamLeafSets;
         if (t.s_write < 0 || (t.s_write >= kStreamWriteVariants && !(lds_form_ok && t.s_write == kStreamByteLds)))
             t.s_write = kStreamWriteDefault;
         if (t.tt_chunk_pct < 10 || t.tt_chunk_pct > 90) t.tt_chunk_pct = 50;
@@ -126,9 +127,9 @@ pf_status Engine::save_tuning(const char* path) const {
 
 // Times the current backend on the sample (positions, depth).
 //  kTuneSinglePass: every tile shape x workgroups-per-CU of the cooperative
-//    kernel, then the stream-ordered form against the best of them, then the
-//    stream-ordered leaf-level kernel's forms (tile shape x waves per SIMD)
-//    and, with the best leaf form, its write-level kernel's forms; kernel
+//    kernel, then the stream-ordered form against the best of them, with the
+//    byte backend's two leaf-level forms and, with the best of these, the
+//    write-level kernel's forms (tile shape x waves per SIMD); kernel
 //    time from HIP events, best of three after a warm-up.
 //  kTuneTable (with a table): the level driver's write-level and leaf-level
 //    workgroups per CU and, when the sample makes the driver chunk, the share
@@ -193,9 +194,9 @@ pf_status Engine::autotune(const pf_pos48* pos, int n, int d, int what) {
             double stream_ms = 1e30;
             for (int pass = 0; pass < 2 && s == PF_OK; pass++) {
                 // the forms of this mode, and for the byte backend its LDS form
-                const int nsv = (pass == 0 ? kStreamVariants : kStreamWriteVariants) + (b == kByte ? 1 : 0);
+                const int forms = pass == 0 ? 1 : kStreamWriteVariants, nsv = forms + (b == kByte ? 1 : 0);
                 for (int i = 0; i < nsv; i++) {
-                    const int v = i < (pass == 0 ? kStreamVariants : kStreamWriteVariants) ? i : kStreamByteLds;
+                    const int v = i >= forms ? kStreamByteLds : pass == 0 ? kStreamLeafSets : i;
                     if (pass == 0) tune[b].s_leaf = v; else tune[b].s_write = v;
                     apply_tuning();
                     double ms = 0;
