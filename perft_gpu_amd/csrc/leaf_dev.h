@@ -9,6 +9,9 @@
 
 namespace pf {
 
+// A value that is the same in all lanes, in a scalar register.
+__device__ __forceinline__ u32 uniform(u32 x) { return __builtin_amdgcn_readfirstlane(x); }
+
 // Records that a wave's 64 parents hand out: those of which the replies of
 // the opponent's king are missing from the start, the others from the end.
 template <int N>
@@ -24,6 +27,7 @@ struct LeafLds {
     LeafPool<N> pool[WG / 64];
     u32 mv[CAP];  // move | parent << 16
     u32 wtot[WG / 64];
+    u32 more[WG / 64];  // waves with calls left undone
 };
 
 // Collects a wave's records.  Every lane of the wave takes part in each call
@@ -42,7 +46,7 @@ struct LeafEmit {
     __device__ __forceinline__ void operator()(u64 k, u64 f, u32 meta) {
         const u64 mk = __ballot(k != 0), mf = __ballot(f != 0);
         if (!(mk | mf)) return;
-        const u32 ck = __builtin_amdgcn_readfirstlane(nk), cf = __builtin_amdgcn_readfirstlane(nf);
+        const u32 ck = uniform(nk), cf = uniform(nf);
         const u32 ek = ck + (u32)__popcll(mk), ef = cf + (u32)__popcll(mf);
         call++;
         if (call <= done) return;
@@ -69,7 +73,9 @@ struct LeafEmit {
 // Ends with a barrier behind the last use of every LDS array.
 template <bool KING, class SL, int TP, int N, int CAP, int WG>
 __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u32 r1, LeafLds<TP, N, CAP, WG>& s) {
-    const u32 tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    u32 tid = threadIdx.x;
+    pin(tid);  // addresses made from it are made again here, not kept in registers through the tile
+    const u32 lane = tid & 63, wid = uniform(tid >> 6);
     const LeafPool<N>& pool = s.pool[wid];
     u32 cnt = 0;
     for (u32 r = r0 + lane; r < r1; r += 64) cnt += leaf_rec_moves(pool.to[r], pool.meta[r]);
@@ -79,7 +85,7 @@ __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u
     u32 woff = 0, tot = 0;
 #pragma unroll
     for (int w = 0; w < WG / 64; w++) {
-        const u32 t = s.wtot[w];
+        const u32 t = uniform(s.wtot[w]);
         woff += (w < (int)wid) ? t : 0;
         tot += t;
     }
@@ -115,7 +121,9 @@ template <class SL, int TP, int N, int CAP, int WG>
 __device__ __forceinline__ void leaf_tile(const SL& sl, const u32 np, LeafLds<TP, N, CAP, WG>& s) {
     static_assert(TP == WG, "one parent per thread");
     static_assert(N >= 128, "one call of a whole wave fits");
-    const u32 tid = threadIdx.x, wid = tid >> 6;
+    u32 tid = threadIdx.x;
+    pin(tid);
+    const u32 wid = uniform(tid >> 6);
     LeafEmit<N> e{&s.pool[wid], (tid & 63) << kLeafMetaBits, 0, 0, 0, 0, false};
     const bool work = (wid << 6) < np;  // of the wave
     bool again = false;
@@ -126,8 +134,13 @@ __device__ __forceinline__ void leaf_tile(const SL& sl, const u32 np, LeafLds<TP
             const u32 sum = leaf_sum(s.b[tid], sl, e);
             if (!again) s.sum[tid] = sum;
         }
-        again = __syncthreads_or(e.more);
+        if ((tid & 63) == 0) s.more[wid] = e.more;
         leaf_records<false>(sl, N - e.nf, N, s);
+        // (read between barriers, so that no wave writes the next round's yet)
+        u32 m = 0;
+#pragma unroll
+        for (int w = 0; w < WG / 64; w++) m |= s.more[w];
+        again = uniform(m) != 0;
         leaf_records<true>(sl, 0, e.nk, s);
     } while (again);
 }

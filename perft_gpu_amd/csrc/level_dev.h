@@ -74,6 +74,7 @@ struct TileLds {
     u32 mv[CAP];
     u32 wtot[WG / 64];
     unsigned long long red[WG / 64];
+    u32 one[WG / 64];  // waves whose parents all have the tile's first root
     u32 tile, base, ok;
 };
 static_assert(sizeof(TileLds<kByteLdsTP, kByteLdsCap, kByteLdsWG>) + kByteLds + 128 <= 160 * 1024,
@@ -96,6 +97,34 @@ struct TileQueue {
         return ntiles > gridDim.x ? gridDim.x + atomicAdd(ctr, 1u) : ntiles;
     }
 };
+
+// sums[root[i]] += ps of thread i < np: one atomic when the tile has a single
+// root (the common case), else one per run of equal roots in each wave.
+template <int W>
+__device__ __forceinline__ void add_tile_sums(unsigned long long* sums, const u32* root, const u32 ps, const u32 np,
+                                              unsigned long long (&red)[W], u32 (&one)[W]) {
+    const u32 tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r0 = root[0];
+    const bool all = __all(tid >= np || root[tid] == r0);
+    const unsigned long long v = wave_sum64((unsigned long long)ps);
+    if (lane == 0) {
+        red[wid] = v;
+        one[wid] = all;
+    }
+    __syncthreads();
+    u32 uni = 1;
+#pragma unroll
+    for (int w = 0; w < W; w++) uni &= one[w];
+    if (uni) {
+        if (tid == 0) {
+            unsigned long long t = 0;
+#pragma unroll
+            for (int w = 0; w < W; w++) t += red[w];
+            if (t) atomicAdd(&sums[r0], t);
+        }
+    } else {
+        wave_run_add(tid < np ? &sums[root[tid]] : nullptr, ps);
+    }
+}
 
 // Process every tile of one level (tiles come from a.tile_ctr).
 template <class SL, int TP, int CAP, int WG>
@@ -169,9 +198,8 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
         }
 
         const u32 ps = ((u32)tid < np) ? s.sum[tid] : 0u;
-        const u32 r0 = s.root[0];
-        const int uni = __syncthreads_and(((u32)tid >= np) || (s.root[tid < TP ? tid : 0] == r0));
-        if (uni || a.total) {
+        if (a.root_sums) add_tile_sums(a.root_sums, s.root, ps, np, s.red, s.one);
+        if (a.total) {
             const unsigned long long v = wave_sum64((unsigned long long)ps);
             if (lane == 0) s.red[wid] = v;
             __syncthreads();
@@ -179,11 +207,9 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
                 unsigned long long t = 0;
 #pragma unroll
                 for (int w = 0; w < WG / 64; w++) t += s.red[w];
-                if (t && a.total) atomicAdd(a.total, t);
-                if (t && uni && a.root_sums) atomicAdd(&a.root_sums[r0], t);
+                if (t) atomicAdd(a.total, t);
             }
         }
-        if (!uni && a.root_sums) wave_run_add((u32)tid < np ? &a.root_sums[s.root[tid]] : nullptr, ps);
         __syncthreads();
     }
 }
@@ -204,6 +230,7 @@ struct LeafLevelLds {
     LeafLds<256, 640, 1280, kWG> t;
     u32 root[256];
     unsigned long long red[kWG / 64];
+    u32 one[kWG / 64];  // waves whose parents all have the tile's first root
     u32 tile;
 };
 
@@ -226,20 +253,7 @@ __device__ __forceinline__ void leaf_level(const SL& sl, const LevelArgs& a, Lea
         __syncthreads();
         leaf_tile(sl, np, s.t);
         const u32 ps = tid < np ? s.t.sum[tid] : 0u;
-        const u32 r0 = s.root[0];
-        if (__syncthreads_and(tid >= np || s.root[tid] == r0)) {
-            const unsigned long long v = wave_sum64((unsigned long long)ps);
-            if (lane == 0) s.red[wid] = v;
-            __syncthreads();
-            if (tid == 0) {
-                unsigned long long t = 0;
-#pragma unroll
-                for (int w = 0; w < kWG / 64; w++) t += s.red[w];
-                if (t) atomicAdd(&a.root_sums[r0], t);
-            }
-        } else {
-            wave_run_add(tid < np ? &a.root_sums[s.root[tid]] : nullptr, ps);
-        }
+        add_tile_sums(a.root_sums, s.root, ps, np, s.red, s.one);
         __syncthreads();
     }
 }

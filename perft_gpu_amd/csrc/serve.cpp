@@ -14,15 +14,17 @@
 // stack, so that it can advance one GPU action at a time.
 //
 // One scheduler step = one replay of a captured graph:
-//   H2D of the step table's host part -> start kernel (zeroes the segment
+//   fetch kernel (the step table's host part) -> start kernel (zeroes the segment
 //   outcomes; new requests: table probe at full depth, move count; empties
 //   the duplicate tables and block sums of this step's write segments) ->
 //   step kernel (the write and leaf levels of every active job in one
 //   persistent launch over two tile queues; duplicates are listed as they are
 //   made) -> up to kUpRounds upsweep kernels (finished levels of every job,
 //   each round the levels just above the previous round's; one graph per
-//   round count) -> D2H of the table's device part: per-segment outcomes,
-//   slot accumulators, table counters.
+//   round count) -> post kernel (the table's device part to the host:
+//   per-segment outcomes, slot accumulators, table counters).
+// A small step (tt_kernels.h) has one launch for fetch and start and one for
+// its upsweeps and outcomes.
 // Requests that arrive while a step runs join the next step; their work
 // overlaps on the device with everyone else's.  All jobs share the lockless
 // transposition table.
@@ -112,21 +114,19 @@ pf_status Server::start() {
     return PF_OK;
 }
 
-// One graph per form of the mixed launch (fine), presence of late leaf passes
-// (late) and number of upsweep rounds (0..kUpRounds): a step replays the one
+// One graph per form of the step, presence of late leaf passes (late) and
+// number of upsweep rounds (0..kUpRounds): a step replays the one
 // that fits it, so a small step does not pay for launches it leaves empty.
-pf_status Server::build_graph(int fine, int late, int rounds) {
+pf_status Server::build_graph(StepForm form, int late, int rounds) {
     hipStream_t st = e_.stream;
     if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) return PF_EDEVICE;
     // the used part of the host's table in, the outcomes (segments, roots,
     // slot accumulators, table counters) out, each by a kernel that reads or
     // writes the coherent host table: no copy node between the host and the
     // step, and a small step moves only what it uses
-    hipError_t e = launch_fetch_step(d_tab_, h_dev_, st);
-    if (e == hipSuccess)
-        e = launch_step(e_.backend, e_.d_tab, e_.d_z, d_tab_, e_.d_tt, e_.tt_buckets ? e_.tt_mask_word() : 0, grid_,
-                        up_grid_, rounds, fine, late, st);
-    if (e == hipSuccess) e = launch_post_step(d_tab_, h_dev_, (u32)max_jobs_, st);
+    const hipError_t e = launch_step(e_.backend, e_.d_tab, e_.d_z, d_tab_, h_dev_, e_.d_tt,
+                                     e_.tt_buckets ? e_.tt_mask_word() : 0, grid_, up_grid_, rounds, form, late,
+                                     (u32)max_jobs_, st);
     // the capture is ended whatever happened inside it, so the stream leaves capture mode
     hipGraph_t g = nullptr;
     const hipError_t ee = hipStreamEndCapture(st, &g);
@@ -134,8 +134,8 @@ pf_status Server::build_graph(int fine, int late, int rounds) {
         if (g) hipGraphDestroy(g);
         return PF_EDEVICE;
     }
-    graph_[fine][late][rounds] = g;
-    if (hipGraphInstantiate(&exec_[fine][late][rounds], g, nullptr, nullptr, 0) != hipSuccess) return PF_EDEVICE;
+    graph_[form][late][rounds] = g;
+    if (hipGraphInstantiate(&exec_[form][late][rounds], g, nullptr, nullptr, 0) != hipSuccess) return PF_EDEVICE;
     return PF_OK;
 }
 
@@ -170,9 +170,9 @@ void Server::idle_spin() {
 // Workgroups of the mixed step launch that start on the write tiles: a share
 // of the workgroups that get a tile (those past the step's tile count leave
 // at once) proportional to the write tiles' part of the step's work, a write
-// tile costing about as much as kWriteTileCost leaf tiles (C5's 4096
-// positions at perft 6 write 1.1e10 children/s and count 5.1e10 in leaf
-// passes).  Whichever queue empties first, its workgroups move to the other.
+// tile costing about as much as kWriteTileCost leaf tiles (a leaf tile of 256
+// parents by sets takes as long as one of 112 move by move did: C5's 4096
+// positions at perft 6 wrote 1.1e10 children/s and counted 5.1e10 in those).  Whichever queue empties first, its workgroups move to the other.
 static constexpr double kWriteTileCost = 4.6;
 u32 Server::mix_write_wgs(u32 write_tiles, u32 leaf_tiles) const {
     if (!write_tiles) return 0;
@@ -194,7 +194,7 @@ void Server::stop() {
         std::lock_guard<std::mutex> g(mu_);
         running_ = false;
     }
-    for (int f = 0; f < 2; f++)
+    for (int f = 0; f < kStepForms; f++)
         for (int l = 0; l < 2; l++)
             for (int r = 0; r <= kUpRounds; r++) {
                 if (exec_[f][l][r]) hipGraphExecDestroy(exec_[f][l][r]);
@@ -624,9 +624,9 @@ bool Server::plan(Job& j) {
 void Server::run() {
     {
         pf_status gs = hipSetDevice(e_.device) == hipSuccess ? PF_OK : PF_EDEVICE;
-        for (int f = 0; f < 2; f++)
+        for (int f = 0; f < kStepForms; f++)
             for (int l = 0; l < 2; l++)
-                for (int r = 0; r <= kUpRounds && gs == PF_OK; r++) gs = build_graph(f, l, r);
+                for (int r = 0; r <= kUpRounds && gs == PF_OK; r++) gs = build_graph((StepForm)f, l, r);
         std::lock_guard<std::mutex> g(mu_);
         graph_status_ = gs;
     }
@@ -771,8 +771,10 @@ void Server::run() {
         t.mix_tp = tp;
         u32 acc_t = 0;
         for (u32 i = 0; i < t.nseg; i++) {
+            // (in the coarse form leaf segments have tiles of their own size)
+            const u32 c = !fine && i >= t.nseg_write ? (u32)kTTLeafParents : tp;
             t.tile_prefix[i] = acc_t;
-            acc_t += (t.seg[i].n_in + tp - 1) / tp;
+            acc_t += (t.seg[i].n_in + c - 1) / c;
         }
         t.tile_prefix[t.nseg] = acc_t;
         t.mix_write_wgs = mix_write_wgs(t.tile_prefix[t.nseg_write], acc_t - t.tile_prefix[t.nseg_write]);
@@ -789,12 +791,22 @@ void Server::run() {
         }
         t.up_round[kUpRounds] = t.nup;
         t.up_prefix[t.nup] = acc_u;
+        // a small step (tt_kernels.h); an upsweep whose counts are not known
+        // yet has at most its write's children as items
+        bool small = fine && t.nseg_write <= (u32)kSmallSegs;
+        u64 items = acc_u, fill = 0;
+        for (u32 k = 0; k < t.nlate && small; k++) items += t.seg[t.late_pos[k]].out_cap;
+        for (u32 i = 0; i < t.nseg_write && small; i++)
+            fill += (t.seg[i].dup ? t.seg[i].dup_n : 0) + t.seg[i].bsum_n / 4;
+        for (int r = 0; r < kUpRounds; r++) small = small && t.up_round[r + 1] - t.up_round[r] <= (u32)kSmallUps;
+        small = small && items <= kSmallItems && fill <= kSmallFill;
+        const StepForm form = small ? kStepSmall : fine ? kStepFine : kStepCoarse;
         const double t0 = now_s();
         int rounds = 0;  // rounds are filled in order: round r + 1 only after round r
         while (rounds < kUpRounds && t.up_round[rounds + 1] > t.up_round[rounds]) rounds++;
         t.seq = ++seq_;
         const bool ok =
-            hipGraphLaunch(exec_[fine][t.nlate > 0][rounds], e_.stream) == hipSuccess && wait_word(&h_tab_->done, t.seq);
+            hipGraphLaunch(exec_[form][t.nlate > 0][rounds], e_.stream) == hipSuccess && wait_word(&h_tab_->done, t.seq);
         const double t1 = now_s();
         {
             std::lock_guard<std::mutex> g(mu_);

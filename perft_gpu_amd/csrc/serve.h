@@ -65,7 +65,7 @@ class Server {
     void finish(Job& j, u64 nodes, int status);
     char* take(Job& j, u64 bytes);
     bool alloc_level(Job& j, u64 n, Engine::TLevel* lv);
-    pf_status build_graph(int fine, int late, int rounds);
+    pf_status build_graph(StepForm form, int late, int rounds);
     bool wait_word(const u32* w, u32 v);
     void idle_spin();
     u32 mix_write_wgs(u32 write_tiles, u32 leaf_tiles) const;
@@ -112,8 +112,8 @@ class Server {
     u64 rb_cap_ = 0;
     u32 late_src_[kMaxLate] = {};  // their write segments (indices before the reordering)
     // by tiling (1: fine), late leaf launch (1: recorded), then upsweep rounds
-    hipGraph_t graph_[2][2][kUpRounds + 1] = {};
-    hipGraphExec_t exec_[2][2][kUpRounds + 1] = {};
+    hipGraph_t graph_[kStepForms][2][kUpRounds + 1] = {};
+    hipGraphExec_t exec_[kStepForms][2][kUpRounds + 1] = {};
     u64 steps_ = 0, segs_ = 0, dups_ = 0;
     double busy_ = 0;
 };

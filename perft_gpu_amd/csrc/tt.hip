@@ -17,6 +17,7 @@
 //     in the table (calcPerftNFromPerftNminus1_hash128b, perft_bb.h:854-961)
 #include <hip/hip_runtime.h>
 
+#include "leaf_dev.h"
 #include "tt_kernels.h"
 #include "wave.h"
 
@@ -35,17 +36,9 @@ static_assert(kTTP * 218 <= kTTMaxWin * kTCAP, "a tile's moves fit kTTMaxWin win
 // the time: ask for at least this many resident waves per SIMD (register
 // budget 512 / waves) so that more of that latency is hidden.
 constexpr int kTTWaves = 4;
-// The level driver's leaf kernel is built for five waves per SIMD (it spills
-// 40 B per lane for Kogge-Stone): C3 perft 8 0.0879 -> 0.0868 s and C5
-// 2.189 -> 2.162 s against four waves without spills.
-constexpr int kTTLeafWaves = 5;
-// The serving step's mixed launch (write and leaf tiles at once) is built for
-// five too: 96 VGPRs, 96 B per lane of spills (none in the leaf loop), five
-// workgroups per CU.  On the 6,018-request serving stream submitted at once:
-// 7.60e12 leaves/s for the write and leaf launches one after the other,
-// 7.96e12 mixed at four waves, 8.04-8.12e12 at five, 8.36-8.40e12 once a tile
-// is taken with one atomic.
-constexpr int kTTMixedWaves = 5;
+// Kernels with a leaf pass by sets (leaf.h) are built for three: it takes 168
+// VGPRs.
+constexpr int kTTLeafWaves = 3;
 
 __device__ __forceinline__ bool tt_probe(const uint4* tt, u64 mask, u64 k1, u64 k2, int depth, u64* val) {
     const uint4* bkt = tt + 2 * tt_bucket(k1, depth, mask);
@@ -318,7 +311,7 @@ __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTa
             if ((u32)tid < np) {
                 const Board b = a.in[p0 + tid];
                 s.b[tid] = b;
-                s.root[tid] = a.in_root[p0 + tid];
+                if (a.mode == kWrite) s.root[tid] = a.in_root[p0 + tid];
                 if (a.tt) {
                     s.k1[tid] = a.in_k1[p0 + tid];
                     s.k2[tid] = a.in_k2[p0 + tid];
@@ -392,6 +385,82 @@ __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTa
     }
 }
 
+// Leaf passes: tiles of kTTLeafParents parents by sets, or smaller ones move by
+// move (tt_tile) where a level has fewer than kLeafSetsMinParents parents per
+// workgroup.  One workgroup's LDS holds either a table tile or a leaf tile.
+// The leaf children are not made and counted one by one (841 vector
+// instructions each) but summed by sets: 256 high-mobility positions at perft 6
+// 117.9 -> 68.6 ms, one middlegame position at perft 8 91 -> 61 ms, a burst of
+// 200 requests 40.3 -> 31.4 ms, same results.
+using TTLeafLds = LeafLds<kTTLeafParents, 640, 1280, kTWG>;
+union TTAnyLds {
+    TTLds w;
+    TTLeafLds l;
+};
+
+// acc[i] += perft 2 of in[i] for i < np <= kTTLeafParents.  Every thread of the
+// block calls it; it ends with a barrier.
+template <class SL>
+__device__ __forceinline__ void tt_leaf_sets(const SL& sl, const Board* in, unsigned long long* acc, const u32 np,
+                                             TTLeafLds& s) {
+    const u32 tid = threadIdx.x;
+    s.b[tid] = tid < np ? in[tid] : Board{};
+    __syncthreads();
+    leaf_tile(sl, np, s);
+    if (tid < np) acc[tid] += s.sum[tid];
+    __syncthreads();
+}
+
+// The c-th range of tp parents of a segment as arguments of their own.
+__device__ __forceinline__ TTArgs tt_range(const TTArgs& a, const u32 c, const u32 tp) {
+    const u32 c0 = c * tp;
+    TTArgs f = a;
+    f.in += c0;
+    f.in_root += c0;
+    f.in_acc += c0;
+    f.in_base += c0;
+    if (f.in_k1) {
+        f.in_k1 += c0;
+        f.in_k2 += c0;
+    }
+    f.n_in = min(tp, a.n_in - c0);
+    return f;
+}
+
+// Leaf range c, of tp parents, of n parents and their accumulators.
+template <class SL>
+__device__ __forceinline__ void tt_leaf_range(const SL& sl, const Board* in, unsigned long long* acc, const u32 n,
+                                              const u32 c, const u32 tp, TTAnyLds& s) {
+    const u32 c0 = c * tp, np = min(tp, n - c0);
+    if (tp >= kLeafSetsMinParents) {
+        tt_leaf_sets(sl, in + c0, acc + c0, np, s.l);
+    } else {
+        TTArgs f = {};
+        f.in = in + c0;
+        f.in_acc = acc + c0;
+        f.n_in = np;
+        f.mode = kLeaf;
+        tt_tile(sl, f, 0, nullptr, s.w);
+    }
+}
+
+// A whole leaf level on the launch's workgroups: a workgroup's own index is
+// its first range, the counter gives the ranges past the grid.
+template <class SL>
+__device__ __forceinline__ void tt_leaf_level(const SL& sl, const Board* in, unsigned long long* acc, const u32 n,
+                                              u32* ctr, u32* s_tile, TTAnyLds& s) {
+    const u32 tp = level_tile_parents(n, gridDim.x, kTTLeafParents);
+    const u32 ntiles = (n + tp - 1) / tp;
+    for (u32 tile = blockIdx.x; tile < ntiles;) {
+        tt_leaf_range(sl, in, acc, n, tile, tp, s);
+        if (ntiles <= gridDim.x) break;
+        if (threadIdx.x == 0) *s_tile = gridDim.x + atomicAdd(ctr, 1u);
+        __syncthreads();
+        tile = __builtin_amdgcn_readfirstlane(*s_tile);
+        __syncthreads();
+    }
+}
+
 template <class SL>
 __device__ void expand_tt_level(const SL& sl, const TTArgs& a, const ZTables* zt, TTLds& s) {
     const u32 ntiles = (a.n_in + kTTP - 1) / kTTP;
@@ -405,15 +474,22 @@ __device__ void expand_tt_level(const SL& sl, const TTArgs& a, const ZTables* zt
     }
 }
 
-// One kernel per mode: with the mode known at compile time the leaf kernel
-// carries none of the write pass, and is built for kTTLeafWaves waves per SIMD.
-template <int B, int M>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(M == kLeaf ? kTTLeafWaves : kTTWaves)))
+// One kernel per mode: the write kernel carries no leaf pass.
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTWaves)))
 void k_expand_tt(const SliderTables* tabs, const ZTables* zt, TTArgs a) {
     __shared__ TTLds s;
     const auto sl = SlOf<B>::make(tabs);
-    a.mode = M;
+    a.mode = kWrite;
     expand_tt_level(sl, a, zt, s);
+}
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves)))
+void k_expand_tt_leaf(const SliderTables* tabs, TTArgs a) {
+    __shared__ TTAnyLds s;
+    __shared__ u32 s_tile;
+    const auto sl = SlOf<B>::make(tabs);
+    tt_leaf_level(sl, a.in, a.in_acc, a.n_in, a.tile_ctr, &s_tile, s);
 }
 
 // Roots: keys were computed on the host; probe at the full depth, count moves.
@@ -460,11 +536,17 @@ __device__ __forceinline__ u32 up_items(const UpSeg& u) {
 // its exact count to its parent and is stored in the table; n <= k < n + ndup
 // is duplicate k - n, which adds the count of the node that claimed its slot.
 // The addition is returned in (*dst, *v) for wave_run_add.  Returns 1 for a
-// store.
+// store.  FRESH: the counts may have been added in this same launch, so they
+// are read where the atomics left them.
+template <bool FRESH>
+__device__ __forceinline__ unsigned long long up_count(const unsigned long long* p) {
+    return FRESH ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+}
+template <bool FRESH>
 __device__ __forceinline__ u32 upsweep_item(const UpSeg& u, u32 n, u32 k, uint4* tt, u64 mask,
                                             unsigned long long** dst, unsigned long long* v) {
     if (k < n) {
-        *v = u.acc[k];
+        *v = up_count<FRESH>(&u.acc[k]);
         *dst = u.parent_acc ? &u.parent_acc[u.parent[k]] : nullptr;
         if (tt && u.depth >= kMinTTDepth) {
             tt_store(tt, mask, u.k1[k], u.k2[k], u.depth, *v);
@@ -475,7 +557,7 @@ __device__ __forceinline__ u32 upsweep_item(const UpSeg& u, u32 n, u32 k, uint4*
     const u32 d = k - n;
     if (u.parent_acc) {
         const u32 c = (u32)u.dup[u.dup_slot[d]].val;
-        *v = u.acc[c];
+        *v = up_count<FRESH>(&u.acc[c]);
         *dst = &u.parent_acc[u.dup_par[d]];
     }
     return 0;
@@ -485,7 +567,7 @@ __global__ __launch_bounds__(256) void k_upsweep(UpSeg u, uint4* tt, u64 mask, u
     const u32 i = blockIdx.x * 256 + threadIdx.x;
     unsigned long long st = 0, v = 0;
     unsigned long long* dst = nullptr;
-    if (i < u.n + u.ndup) st = upsweep_item(u, u.n, i, tt, mask, &dst, &v);
+    if (i < u.n + u.ndup) st = upsweep_item<false>(u, u.n, i, tt, mask, &dst, &v);
     wave_run_add(dst, v);
     if (stores) {
         st = wave_sum64(st);
@@ -509,51 +591,51 @@ __device__ __forceinline__ TTArgs uniform_args(const TTArgs& src) {
     return a;
 }
 
-// Tiles of the step's expand segments form a queue (StepTable::tile_prefix);
-// a block copies its segment's arguments to LDS and runs the tile.  Segments
-// of different jobs touch disjoint memory except the lockless table.
-// W: the waves per SIMD it is built for; M = kWrite runs the table's write
-// segments [0, nseg_write) and M = kLeaf its leaf segments [nseg_write,
-// nseg), each without the other mode's code (as in k_expand_tt).
-template <int B, int W, int M>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void k_step(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
+// A segment's arguments into LDS, a word per thread.
+__device__ __forceinline__ void copy_words(TTArgs& dst, const TTArgs& src) {
+    static_assert(sizeof(TTArgs) / 4 <= kTWG, "one word per thread");
+    if (threadIdx.x < sizeof(TTArgs) / 4)
+        reinterpret_cast<u32*>(&dst)[threadIdx.x] = reinterpret_cast<const u32*>(&src)[threadIdx.x];
+}
+
+template <class T>
+__device__ __forceinline__ T* uniform_ptr(T* p) {
+    const u64 v = reinterpret_cast<u64>(p);
+    const u32 lo = __builtin_amdgcn_readfirstlane((u32)v), hi = __builtin_amdgcn_readfirstlane((u32)(v >> 32));
+    return reinterpret_cast<T*>(((u64)hi << 32) | lo);
+}
+
+// The planned pass's write launch: its one segment's tiles from a queue.
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTWaves))) void k_step_write(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
     __shared__ TTLds s;
     __shared__ TTArgs sa;
-    __shared__ u32 s_tile, s_seg;
+    __shared__ u32 s_tile;
     const auto sl = SlOf<B>::make(tabs);
-    const u32 s_lo = (M == kLeaf) ? t->nseg_write : 0u, s_hi = (M == kWrite) ? t->nseg_write : t->nseg;
-    const u32 first = t->tile_prefix[s_lo], total = t->tile_prefix[s_hi];
-    if (M == kWrite && t->fuse_leaf) return;  // the fused launch runs this level
-    if (blockIdx.x >= total - first) return;  // more workgroups than tiles: the others drain the queue
-    u32* const ctr = (M == kLeaf) ? &t->tile_ctr2 : &t->tile_ctr;
-    u32 cur = 0xFFFFFFFFu;
+    const u32 total = t->tile_prefix[t->nseg_write];
+    if (t->fuse_leaf) return;  // the fused launch runs this level
+    if (blockIdx.x >= total) return;  // more workgroups than tiles: the others drain the queue
+    copy_words(sa, t->seg[0]);
+    __syncthreads();
+    TTArgs a = uniform_args(sa);
+    a.mode = kWrite;
     for (;;) {
-        if (threadIdx.x == 0) {
-            const u32 g = first + atomicAdd(ctr, 1u);
-            u32 seg = s_lo;
-            if (g < total) {
-                u32 lo = s_lo, hi = s_hi;  // largest seg with tile_prefix[seg] <= g
-                while (hi - lo > 1) {
-                    const u32 mid = (lo + hi) >> 1;
-                    if (t->tile_prefix[mid] <= g) lo = mid; else hi = mid;
-                }
-                seg = lo;
-            }
-            s_tile = g;
-            s_seg = seg;
-        }
+        if (threadIdx.x == 0) s_tile = atomicAdd(&t->tile_ctr, 1u);
         __syncthreads();
-        const u32 g = s_tile, seg = s_seg;
+        const u32 g = s_tile;
         if (g >= total) break;
-        if (seg != cur) {
-            if (threadIdx.x == 0) sa = t->seg[seg];
-            cur = seg;
-        }
-        __syncthreads();
-        TTArgs a = uniform_args(sa);
-        a.mode = M;
-        tt_tile(sl, a, g - t->tile_prefix[seg], zt, s);
+        tt_tile(sl, a, g, zt, s);
     }
+}
+
+// The planned pass's leaf launch.
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_leaf(const SliderTables* tabs, StepTable* t) {
+    __shared__ TTAnyLds s;
+    __shared__ u32 s_tile;
+    if (!t->nseg) return;  // the level ran fused, or overflowed
+    const auto sl = SlOf<B>::make(tabs);
+    tt_leaf_level(sl, t->seg[0].in, t->seg[0].in_acc, t->seg[0].n_in, &t->tile_ctr2, &s_tile, s);
 }
 
 // The planned pass's last write level and its leaf pass in one launch (its
@@ -565,44 +647,44 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
 // in the caches.  Workgroups are in different phases at any time, so the
 // write tiles' waits on table and duplicate claims overlap other workgroups'
 // leaf VALU work, where a write launch followed by a leaf launch ran them one
-// after the other: C5's first 2048 positions at perft 6 0.934 -> 0.865 s, C3
-// perft 8 0.080 -> 0.076 s.  The kept children of a tile are the windows'
+// after the other: 256 high-mobility positions at perft 6 71.3 -> 67.5 ms, one
+// middlegame position at perft 8 53.7 -> 51.3 ms.  The kept children of a tile are the windows'
 // reserved ranges (TTLds::wr_base/wr_n), whose accumulators the write just
 // zeroed; the leaf tiles add perft(child, 2) to them.
-template <int B, int W>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void k_step_write_leaf(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
-    __shared__ TTLds s;
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_write_leaf(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
+    __shared__ TTAnyLds s;
     __shared__ TTArgs sa;
     __shared__ u32 s_tile;
+    __shared__ u32 s_nwin, s_base[kTTMaxWin], s_n[kTTMaxWin];
     const auto sl = SlOf<B>::make(tabs);
     const u32 total = t->tile_prefix[1];
     if (!t->fuse_leaf) return;  // the level was written by the write launch; the leaf launch follows
     if (blockIdx.x >= total) return;  // more workgroups than tiles: the others drain the queue
-    if (threadIdx.x == 0) sa = t->seg[0];
-    __syncthreads();
-    TTArgs a = uniform_args(sa);
-    a.mode = kWrite;
-    TTArgs l = {};  // the leaf tiles' arguments: parents are the written children
-    l.mode = kLeaf;
-    l.child_depth = a.child_depth - 1;
-    l.err = a.err;
+    copy_words(sa, t->seg[0]);
     for (;;) {
         if (threadIdx.x == 0) s_tile = atomicAdd(&t->tile_ctr, 1u);
         __syncthreads();
         const u32 g = s_tile;
         if (g >= total) break;
-        tt_tile(sl, a, g, zt, s);  // ends with a barrier: s.nwin and the ranges are final
-        const u32 nwin = s.nwin;
-        __syncthreads();  // every wave has nwin before a leaf tile reuses the tile state
+        {
+            TTArgs a = uniform_args(sa);
+            a.mode = kWrite;
+            tt_tile(sl, a, g, zt, s.w);  // ends with a barrier: the windows' ranges are final
+        }
+        if (threadIdx.x < kTTMaxWin) {  // a leaf tile reuses the tile state
+            s_base[threadIdx.x] = s.w.wr_base[threadIdx.x];
+            s_n[threadIdx.x] = s.w.wr_n[threadIdx.x];
+            if (threadIdx.x == 0) s_nwin = s.w.nwin;
+        }
+        __syncthreads();
+        const u32 nwin = __builtin_amdgcn_readfirstlane(s_nwin);
         for (u32 w = 0; w < nwin; w++) {
-            const u32 rb = s.wr_base[w], rn = s.wr_n[w];
-            for (u32 c0 = 0; c0 < rn; c0 += kTTP) {
-                l.in = a.out + rb + c0;
-                l.in_root = a.out_root + rb + c0;
-                l.in_acc = a.out_acc + rb + c0;
-                l.n_in = min((u32)kTTP, rn - c0);
-                tt_tile(sl, l, 0, zt, s);
-            }
+            const u32 rb = __builtin_amdgcn_readfirstlane(s_base[w]), rn = __builtin_amdgcn_readfirstlane(s_n[w]);
+            const Board* in = uniform_ptr(sa.out) + rb;
+            unsigned long long* acc = uniform_ptr(sa.out_acc) + rb;
+            for (u32 c0 = 0; c0 < rn; c0 += kTTLeafParents)
+                tt_leaf_sets(sl, in + c0, acc + c0, min((u32)kTTLeafParents, rn - c0), s.l);
         }
     }
 }
@@ -616,33 +698,40 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
 // nseg) with tile_ctr2; their bounds are read once, before the loop, and the
 // tile prefix is copied to LDS, so that taking a tile is one atomic and a
 // search in LDS (small steps are latency-bound).
-template <int B, int W, bool F>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void k_step_mixed(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
-    __shared__ TTLds s;
+template <int B, bool F>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_mixed(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
+    __shared__ TTAnyLds s;
     __shared__ TTArgs sa;
     __shared__ u32 s_tile, s_seg;
     __shared__ u32 pre[kMaxSegs + 1];  // the tile prefix, searched for every tile
     const auto sl = SlOf<B>::make(tabs);
     const u32 nw = t->nseg_write, ns = t->nseg;
-    const u32 wt = t->tile_prefix[nw], lt = t->tile_prefix[ns];  // write tiles [0, wt), leaf tiles [wt, lt)
-    if (blockIdx.x >= lt) return;  // more workgroups than tiles: the others drain the queues
-    const u32 tp = F ? t->mix_tp : (u32)kTTP;
-    for (u32 k = threadIdx.x; k <= ns; k += kTWG) pre[k] = t->tile_prefix[k];
+    // (the whole array, so that its loads do not wait for nseg)
+    for (u32 k = threadIdx.x; k <= (u32)kMaxSegs; k += kTWG) pre[k] = t->tile_prefix[k];
     __syncthreads();
-    bool leaf = blockIdx.x >= t->mix_write_wgs;  // thread 0's queue
-    bool moved = false;
+    const u32 wt = uniform(pre[nw]), lt = uniform(pre[ns]);  // write tiles [0, wt), leaf tiles [wt, lt)
+    if (blockIdx.x >= lt) return;  // more workgroups than tiles: no tile of their own, the others drain the queues
+    const u32 tp = F ? t->mix_tp : 0u;
+    // Workgroups [0, w0) start with the write tile of their own index, the
+    // others with the leaf tiles from wt on; the counters give the rest, so a
+    // small step takes no tile by an atomic.
+    const u32 w0 = min(min(t->mix_write_wgs, wt), gridDim.x);
+    bool leaf = blockIdx.x >= w0, moved = false, own = true;  // thread 0's queue
     u32 cur = 0xFFFFFFFFu;
     for (;;) {
         if (threadIdx.x == 0) {
             u32 g = 0xFFFFFFFFu;
             for (;;) {
-                const u32 first = leaf ? wt : 0u, total = leaf ? lt : wt;
-                if (first < total) {
-                    const u32 k = first + atomicAdd(leaf ? &t->tile_ctr2 : &t->tile_ctr, 1u);
-                    if (k < total) {
-                        g = k;
-                        break;
-                    }
+                const u32 end = leaf ? lt : wt;
+                u32 k;
+                if (own) k = leaf ? wt + (blockIdx.x - w0) : blockIdx.x;
+                else if (leaf) k = wt + (gridDim.x - w0);
+                else k = w0;
+                if (!own && k < end) k += atomicAdd(leaf ? &t->tile_ctr2 : &t->tile_ctr, 1u);
+                own = false;
+                if (k < end) {
+                    g = k;
+                    break;
                 }
                 if (moved) break;
                 leaf = !leaf;
@@ -661,29 +750,22 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
             s_seg = seg;
         }
         __syncthreads();
-        const u32 g = s_tile, seg = s_seg;
+        const u32 g = s_tile, seg = uniform(s_seg);
         if (g == 0xFFFFFFFFu) break;
         if (seg != cur) {
-            if (threadIdx.x == 0) sa = t->seg[seg];
+            copy_words(sa, t->seg[seg]);
             cur = seg;
         }
         __syncthreads();
-        const TTArgs a = uniform_args(sa);  // the segment's own mode
-        if (F) {  // tile g - pre[seg] of the segment: its tp parents as a one-tile range
-            const u32 c0 = (g - pre[seg]) * tp;
-            TTArgs f = a;
-            f.in += c0;
-            f.in_root += c0;
-            f.in_acc += c0;
-            f.in_base += c0;
-            if (f.in_k1) {
-                f.in_k1 += c0;
-                f.in_k2 += c0;
-            }
-            f.n_in = min(tp, a.n_in - c0);
-            tt_tile(sl, f, 0, zt, s);
+        const u32 c = uniform(g - pre[seg]);
+        if (seg >= nw) {
+            tt_leaf_range(sl, uniform_ptr(sa.in), uniform_ptr(sa.in_acc), uniform(sa.n_in), c,
+                          F ? tp : (u32)kTTLeafParents, s);
         } else {
-            tt_tile(sl, a, g - pre[seg], zt, s);
+            TTArgs a = uniform_args(sa);
+            a.mode = kWrite;
+            if (F) a = tt_range(a, c, tp);
+            tt_tile(sl, a, F ? 0 : c, zt, s.w);
         }
     }
 }
@@ -693,11 +775,13 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
 // written, counted and upswept in one step.  Each pass's parents are its write
 // segment's children; their number is that write's outcome (none if it
 // overflowed), so the tile prefix is built here, by the first wave.
-template <int B, int W>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void k_step_late(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
-    __shared__ TTLds s;
-    __shared__ u32 pre[kMaxLate + 1];
-    __shared__ u32 s_tile, s_seg, s_tp;
+template <int B>
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_late(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
+    __shared__ TTAnyLds s;
+    __shared__ u32 pre[kMaxLate + 1], s_n[kMaxLate];
+    __shared__ const Board* s_in[kMaxLate];
+    __shared__ unsigned long long* s_acc[kMaxLate];
+    __shared__ u32 s_tile, s_tp;
     const u32 nl = t->nlate;
     if (!nl) return;
     const auto sl = SlOf<B>::make(tabs);
@@ -706,12 +790,16 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
         if (threadIdx.x < nl) {
             const TTArgs& w = t->seg[t->late_pos[threadIdx.x]];
             n = *w.err ? 0u : *w.out_count;
+            // the write's children as parents
+            s_n[threadIdx.x] = n;
+            s_in[threadIdx.x] = w.out;
+            s_acc[threadIdx.x] = w.out_acc;
         }
         // parents per tile: the fewest that still give every tile a workgroup
         // of this launch (these levels are small and wait on the chain of one
         // tile's dependent steps), at most a full tile
-        u32 tp = kTTP;
-        for (u32 c = kFineMinParents; c < (u32)kTTP; c *= 2)
+        u32 tp = kTTLeafParents;
+        for (u32 c = kFineMinParents; c < (u32)kTTLeafParents; c *= 2)
             if (__builtin_amdgcn_readlane(wave_incl_scan((n + c - 1) / c), 63) <= gridDim.x) {
                 tp = c;
                 break;
@@ -724,41 +812,57 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(W))) void 
         }
     }
     __syncthreads();
-    const u32 total = pre[nl], tp = s_tp;
-    if (blockIdx.x >= total) return;  // more workgroups than tiles: the others drain the queue
-    u32 cur = 0xFFFFFFFFu, wn = 0;
-    TTArgs l = {}, wl = {};
-    for (;;) {
-        if (threadIdx.x == 0) {
-            const u32 g = atomicAdd(&t->tile_ctr3, 1u);
-            u32 lo = 0, hi = nl;  // largest k with pre[k] <= g
-            if (g < total)
-                while (hi - lo > 1) {
-                    const u32 mid = (lo + hi) >> 1;
-                    if (pre[mid] <= g) lo = mid; else hi = mid;
-                }
-            s_tile = g;
-            s_seg = lo;
-        }
+    const u32 total = uniform(pre[nl]), tp = uniform(s_tp);
+    // a workgroup's own index is its first tile, the counter gives those past the grid
+    for (u32 g = blockIdx.x; g < total;) {
+        u32 k = 0;
+        while (uniform(pre[k + 1]) <= g) k++;
+        tt_leaf_range(sl, uniform_ptr(s_in[k]), uniform_ptr(s_acc[k]), uniform(s_n[k]), g - uniform(pre[k]), tp, s);
+        if (total <= gridDim.x) break;
+        if (threadIdx.x == 0) s_tile = gridDim.x + atomicAdd(&t->tile_ctr3, 1u);
         __syncthreads();
-        const u32 g = s_tile, k = s_seg;
-        if (g >= total) break;
-        if (k != cur) {  // the write's children as parents (uniform: from LDS and the table)
-            const TTArgs& w = t->seg[t->late_pos[k]];
-            wl = w;
-            wn = *w.out_count;
-            l.mode = kLeaf;
-            l.child_depth = w.child_depth - 1;
-            l.err = w.err;
-            cur = k;
+        g = uniform(s_tile);
+        __syncthreads();
+    }
+}
+
+// Items [first, last) of the segments [s0, s0 + ns), whose item prefix is in
+// LDS, `stride` of them apart per pass of the calling workgroup.
+template <bool FRESH>
+__device__ __forceinline__ void up_loop(const StepTable* __restrict__ t, uint4* tt, u64 mask, const u32 s0,
+                                        const u32 ns, const u32* pre, const u32 last, const u32 first,
+                                        const u32 stride) {
+    unsigned long long stores = 0;
+    // the loop is uniform per wave (wave_run_add needs every lane)
+    for (u32 w = first + (threadIdx.x & ~63u); w < last; w += stride) {
+        const u32 i = w + (threadIdx.x & 63);
+        unsigned long long v = 0;
+        unsigned long long* dst = nullptr;
+        u32 lo = 0;
+        if (i < last) {
+            u32 hi = ns;  // largest segment with pre[lo] <= i
+            while (hi - lo > 1) {
+                const u32 mid = (lo + hi) >> 1;
+                if (pre[mid] <= i) lo = mid; else hi = mid;
+            }
         }
-        // tile g - pre[k] of the level: its tp parents as a one-tile range
-        const u32 c0 = (g - pre[k]) * tp;
-        l.in = wl.out + c0;
-        l.in_root = wl.out_root + c0;
-        l.in_acc = wl.out_acc + c0;
-        l.n_in = min(tp, wn - c0);
-        tt_tile(sl, l, 0, zt, s);
+        // most waves lie in one segment: its arguments then come through
+        // scalar loads, once per wave
+        const u32 lo0 = __builtin_amdgcn_readfirstlane(lo);
+        if (__all(i >= last || lo == lo0)) {
+            if (i < last) {
+                const UpSeg& u = t->up[s0 + lo0];
+                stores += upsweep_item<FRESH>(u, up_nodes(u), i - pre[lo0], tt, mask, &dst, &v);
+            }
+        } else if (i < last) {
+            const UpSeg& u = t->up[s0 + lo];
+            stores += upsweep_item<FRESH>(u, up_nodes(u), i - pre[lo], tt, mask, &dst, &v);
+        }
+        wave_run_add(dst, v);
+    }
+    if (t->stores) {
+        stores = wave_sum64(stores);
+        if ((threadIdx.x & 63) == 0 && stores) atomicAdd(t->stores, stores);
     }
 }
 
@@ -788,38 +892,7 @@ __global__ __launch_bounds__(256) void k_up_step(const StepTable* __restrict__ t
     if (threadIdx.x == 0) pre[ns] = last;
     __syncthreads();
     if (blockIdx.x * 256 >= last) return;  // no item for this workgroup
-    unsigned long long stores = 0;
-    // the loop is uniform per wave (wave_run_add needs every lane)
-    for (u32 w = blockIdx.x * 256 + (threadIdx.x & ~63u); w < last; w += gridDim.x * 256) {
-        const u32 i = w + (threadIdx.x & 63);
-        unsigned long long v = 0;
-        unsigned long long* dst = nullptr;
-        u32 lo = 0;
-        if (i < last) {
-            u32 hi = ns;  // largest segment with pre[lo] <= i
-            while (hi - lo > 1) {
-                const u32 mid = (lo + hi) >> 1;
-                if (pre[mid] <= i) lo = mid; else hi = mid;
-            }
-        }
-        // most waves lie in one segment: its arguments then come through
-        // scalar loads, once per wave
-        const u32 lo0 = __builtin_amdgcn_readfirstlane(lo);
-        if (__all(i >= last || lo == lo0)) {
-            if (i < last) {
-                const UpSeg& u = t->up[s0 + lo0];
-                stores += upsweep_item(u, up_nodes(u), i - pre[lo0], tt, mask, &dst, &v);
-            }
-        } else if (i < last) {
-            const UpSeg& u = t->up[s0 + lo];
-            stores += upsweep_item(u, up_nodes(u), i - pre[lo], tt, mask, &dst, &v);
-        }
-        wave_run_add(dst, v);
-    }
-    if (t->stores) {
-        stores = wave_sum64(stores);
-        if ((threadIdx.x & 63) == 0 && stores) atomicAdd(t->stores, stores);
-    }
+    up_loop<false>(t, tt, mask, s0, ns, pre, last, blockIdx.x * 256, gridDim.x * 256);
 }
 
 // Serving: the step table's host part, read by the GPU from coherent host
@@ -827,16 +900,8 @@ __global__ __launch_bounds__(256) void k_up_step(const StepTable* __restrict__ t
 // the used segments, upsweeps and roots), so that a small step moves about a
 // kilobyte rather than the whole table, and no copy node sits between the
 // host and the step's first kernel.  Copied as 4-byte words.
-__global__ __launch_bounds__(256) void k_fetch_step(StepTable* __restrict__ d, const StepTable* __restrict__ h) {
-    __shared__ u32 hdr[3];
-    if (threadIdx.x == 0) {
-        hdr[0] = h->nseg;
-        hdr[1] = h->nup;
-        hdr[2] = h->nroot;
-    }
-    __syncthreads();
-    // (clamped to the table's capacities, so every word copied lies inside it)
-    const u32 nseg = min(hdr[0], (u32)kMaxSegs), nup = min(hdr[1], (u32)kMaxUps), nroot = min(hdr[2], (u32)kMaxRoots);
+__device__ __forceinline__ void fetch_words(StepTable* __restrict__ d, const StepTable* __restrict__ h, const u32 nseg,
+                                            const u32 nup, const u32 nroot) {
     constexpr u32 kHdr = offsetof(StepTable, tile_prefix) / 4;
     const u32 o_tp = offsetof(StepTable, tile_prefix) / 4, n_tp = nseg + 1;
     const u32 o_ur = offsetof(StepTable, up_round) / 4, n_ur = kUpRounds + 1;
@@ -857,6 +922,17 @@ __global__ __launch_bounds__(256) void k_fetch_step(StepTable* __restrict__ d, c
         dst[w] = src[w];
     }
 }
+__global__ __launch_bounds__(256) void k_fetch_step(StepTable* __restrict__ d, const StepTable* __restrict__ h) {
+    __shared__ u32 hdr[3];
+    if (threadIdx.x == 0) {
+        hdr[0] = h->nseg;
+        hdr[1] = h->nup;
+        hdr[2] = h->nroot;
+    }
+    __syncthreads();
+    // (clamped to the table's capacities, so every word copied lies inside it)
+    fetch_words(d, h, min(hdr[0], (u32)kMaxSegs), min(hdr[1], (u32)kMaxUps), min(hdr[2], (u32)kMaxRoots));
+}
 static_assert(sizeof(TTArgs) % 4 == 0 && sizeof(UpSeg) % 4 == 0 && sizeof(RootSeg) % 4 == 0 &&
                   offsetof(StepTable, tile_prefix) % 4 == 0,
               "the step table is fetched in 4-byte words");
@@ -866,17 +942,41 @@ static_assert(sizeof(TTArgs) % 4 == 0 && sizeof(UpSeg) % 4 == 0 && sizeof(RootSe
 // counters); then, once all of them are visible to the host, the step's
 // number into done, so that the host can wait for the step by watching it.
 // One workgroup.
-__global__ __launch_bounds__(256) void k_post_step(const StepTable* d, StepTable* h, u32 max_jobs) {
+template <int WG, bool FRESH>
+__device__ __forceinline__ void post_step(const StepTable* d, StepTable* h, u32 max_jobs) {
     const u32 nseg = min(d->nseg, (u32)kMaxSegs), nroot = min(d->nroot, (u32)kMaxRoots);
     max_jobs = min(max_jobs, (u32)kMaxRoots);
-    for (u32 i = threadIdx.x; i < nseg; i += 256) h->out[i] = d->out[i];
-    for (u32 i = threadIdx.x; i < nroot; i += 256) h->rout[i] = d->rout[i];
-    for (u32 i = threadIdx.x; i < max_jobs; i += 256) h->acc[i] = d->acc[i];
+    for (u32 i = threadIdx.x; i < nseg; i += WG) h->out[i] = d->out[i];
+    for (u32 i = threadIdx.x; i < nroot; i += WG) h->rout[i] = d->rout[i];
+    for (u32 i = threadIdx.x; i < max_jobs; i += WG) h->acc[i] = up_count<FRESH>(&d->acc[i]);
     if (threadIdx.x < 2) h->stats[threadIdx.x] = d->stats[threadIdx.x];
     __threadfence_system();  // this thread's writes reach the host before the barrier ...
-    __syncthreads();
+    if (WG > 64) __syncthreads();
     if (threadIdx.x == 0)    // ... and so before done
         __hip_atomic_store(&h->done, d->seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ __launch_bounds__(256) void k_post_step(const StepTable* d, StepTable* h, u32 max_jobs) {
+    post_step<256, false>(d, h, max_jobs);
+}
+
+// A small step's upsweep rounds and outcomes in one launch of one workgroup
+// (StepTable's up_round: at most kSmallUps segments a round).
+__global__ __launch_bounds__(kSmallWG) void k_up_post(StepTable* d, StepTable* h, uint4* tt, u64 mask,
+                                                      int rounds, u32 max_jobs) {
+    static_assert(kSmallUps == 64, "one wave builds a round's item prefix");
+    __shared__ u32 pre[kSmallUps + 1];
+    for (int r = 0; r < rounds; r++) {
+        const u32 s0 = d->up_round[r], ns = min(d->up_round[r + 1] - s0, (u32)kSmallUps);
+        if (threadIdx.x < 64) {
+            const u32 incl = wave_incl_scan(threadIdx.x < ns ? up_items(d->up[s0 + threadIdx.x]) : 0u);
+            pre[threadIdx.x + 1] = incl;
+            if (threadIdx.x == 0) pre[0] = 0;
+        }
+        __syncthreads();
+        up_loop<true>(d, tt, mask, s0, ns, pre, pre[ns], 0, kSmallWG);
+        __syncthreads();  // the round's atomics are done
+    }
+    if (threadIdx.x < 64) post_step<64, true>(d, h, max_jobs);  // (one wave: its system fence is the launch's only one)
 }
 
 __global__ void k_post_flag(u32* flag, u32 v) {
@@ -888,13 +988,28 @@ hipError_t launch_post_flag(u32* flag, u32 v, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_fetch_step(StepTable* d, const StepTable* h, hipStream_t s) {
-    hipLaunchKernelGGL(k_fetch_step, dim3(32), dim3(256), 0, s, d, h);
-    return hipGetLastError();
-}
-hipError_t launch_post_step(const StepTable* d, StepTable* h, u32 max_jobs, hipStream_t s) {
-    hipLaunchKernelGGL(k_post_step, dim3(1), dim3(256), 0, s, d, h, max_jobs);
-    return hipGetLastError();
+// A new request: probed at full depth, else its moves counted.
+template <class SL>
+__device__ __forceinline__ void step_root(const SL& sl, const RootSeg& r, const uint4* tt, u64 mask, RootOut* out) {
+    const Board b = r.b;
+    *r.dst_w = r.word;
+    if (tt) {
+        *r.dst_k1 = r.k1;
+        *r.dst_k2 = r.k2;
+    }
+    u64 v = 0;
+    if (tt && r.depth >= kMinTTDepth && tt_probe(tt, mask, r.k1, r.k2, r.depth, &v)) {
+        *r.acc = v;
+        *r.dst_b = with_count(b, 0);  // answered: nothing below it is expanded
+        out->hit = 1;
+        out->count = 0;
+    } else {
+        const u32 c = count_moves(b, sl);
+        *r.dst_b = with_count(b, c);
+        *r.acc = (r.depth == 1) ? c : 0;
+        out->hit = 0;
+        out->count = c;
+    }
 }
 
 // Start of a step: the step's segment outcomes zeroed, new requests (table
@@ -909,28 +1024,7 @@ __global__ __launch_bounds__(256) void k_pre_step(const SliderTables* tabs, Step
     const auto sl = SlOf<B>::make(tabs);
     const u32 gi = blockIdx.x * 256 + threadIdx.x;
     if (gi < t->nseg) t->out[gi] = SegOut{};
-    if (gi < t->nroot) {
-        const RootSeg& r = t->root[gi];
-        const Board b = r.b;
-        *r.dst_w = r.word;
-        if (tt) {
-            *r.dst_k1 = r.k1;
-            *r.dst_k2 = r.k2;
-        }
-        u64 v = 0;
-        if (tt && r.depth >= kMinTTDepth && tt_probe(tt, mask, r.k1, r.k2, r.depth, &v)) {
-            *r.acc = v;
-            *r.dst_b = with_count(b, 0);  // answered: nothing below it is expanded
-            t->rout[gi].hit = 1;
-            t->rout[gi].count = 0;
-        } else {
-            const u32 c = count_moves(b, sl);
-            *r.dst_b = with_count(b, c);
-            *r.acc = (r.depth == 1) ? c : 0;
-            t->rout[gi].hit = 0;
-            t->rout[gi].count = c;
-        }
-    }
+    if (gi < t->nroot) step_root(sl, t->root[gi], tt, mask, &t->rout[gi]);
     const u64 stride = (u64)gridDim.x * 256;
     const u32 nw = t->nseg_write;  // leaf segments [nw, nseg) have no tables
     for (u32 si = 0; si < nw; si++) {
@@ -942,19 +1036,53 @@ __global__ __launch_bounds__(256) void k_pre_step(const SliderTables* tabs, Step
     }
 }
 
+// A small step's fetch and start in one launch (StepTable: at most
+// kSmallSegs write segments).  What the start reads it reads from the host's
+// table, as another workgroup may be the one that copies it.
+template <int B>
+__global__ __launch_bounds__(256) void k_fetch_pre(const SliderTables* tabs, StepTable* __restrict__ d,
+                                                   const StepTable* __restrict__ h, const uint4* tt, u64 mask) {
+    __shared__ u32 hdr[4];
+    __shared__ DupEntry* s_dup[kSmallSegs];
+    __shared__ u32* s_bsum[kSmallSegs];
+    __shared__ u64 s_dn[kSmallSegs];
+    __shared__ u32 s_bn[kSmallSegs];
+    const u32 tid = threadIdx.x;
+    if (tid == 0) hdr[0] = h->nseg;
+    if (tid == 1) hdr[1] = h->nup;
+    if (tid == 2) hdr[2] = h->nroot;
+    if (tid == 3) hdr[3] = h->nseg_write;
+    if (tid >= 64 && tid < 64 + (u32)kSmallSegs) {  // (entries past nseg_write are not used)
+        const TTArgs& a = h->seg[tid - 64];
+        s_dup[tid - 64] = a.dup;
+        s_dn[tid - 64] = a.dup_n;
+        s_bsum[tid - 64] = a.out_bsum;
+        s_bn[tid - 64] = a.bsum_n;
+    }
+    __syncthreads();
+    const u32 nseg = min(hdr[0], (u32)kMaxSegs), nroot = min(hdr[2], (u32)kMaxRoots);
+    const u32 gi = blockIdx.x * 256 + tid;
+    if (gi < nseg) d->out[gi] = SegOut{};
+    if (gi < nroot) step_root(SlOf<B>::make(tabs), h->root[gi], tt, mask, &d->rout[gi]);
+    fetch_words(d, h, nseg, min(hdr[1], (u32)kMaxUps), nroot);
+    const u32 stride = gridDim.x * 256, nw = min(hdr[3], (u32)kSmallSegs);
+    for (u32 si = 0; si < nw; si++) {
+        if (s_bsum[si])
+            for (u32 i = gi; i < s_bn[si]; i += stride) s_bsum[si][i] = 0;
+        if (s_dup[si])
+            for (u64 i = gi; i < s_dn[si]; i += stride) s_dup[si][i] = DupEntry{0, 0};
+    }
+}
+
 // Most resident workgroups per CU of the planned pass's step kernels.
 int step_max_bpc(int backend, int leaf) {
     const void* f;
     if (leaf)
-        f = backend == kKS ? (const void*)&k_step<kKS, kTTLeafWaves, kLeaf>
-            : backend == kPlain ? (const void*)&k_step<kPlain, kTTLeafWaves, kLeaf>
-            : backend == kFancy ? (const void*)&k_step<kFancy, kTTLeafWaves, kLeaf>
-                                : (const void*)&k_step<kByte, kTTLeafWaves, kLeaf>;
+        f = backend == kKS ? (const void*)&k_step_leaf<kKS> : backend == kPlain ? (const void*)&k_step_leaf<kPlain>
+            : backend == kFancy ? (const void*)&k_step_leaf<kFancy> : (const void*)&k_step_leaf<kByte>;
     else
-        f = backend == kKS ? (const void*)&k_step<kKS, kTTWaves, kWrite>
-            : backend == kPlain ? (const void*)&k_step<kPlain, kTTWaves, kWrite>
-            : backend == kFancy ? (const void*)&k_step<kFancy, kTTWaves, kWrite>
-                                : (const void*)&k_step<kByte, kTTWaves, kWrite>;
+        f = backend == kKS ? (const void*)&k_step_write<kKS> : backend == kPlain ? (const void*)&k_step_write<kPlain>
+            : backend == kFancy ? (const void*)&k_step_write<kFancy> : (const void*)&k_step_write<kByte>;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kTWG, 0) != hipSuccess || per_cu < 1) {
         (void)hipGetLastError();  // a failed query must not surface as a later call's error
@@ -965,10 +1093,10 @@ int step_max_bpc(int backend, int leaf) {
 
 // The serving step's mixed kernel: its most resident workgroups per CU x CUs.
 int step_grid(int backend, int n_cu) {
-    const void* f = backend == kKS ? (const void*)&k_step_mixed<kKS, kTTMixedWaves, false>
-                    : backend == kPlain ? (const void*)&k_step_mixed<kPlain, kTTMixedWaves, false>
-                    : backend == kFancy ? (const void*)&k_step_mixed<kFancy, kTTMixedWaves, false>
-                                        : (const void*)&k_step_mixed<kByte, kTTMixedWaves, false>;
+    const void* f = backend == kKS ? (const void*)&k_step_mixed<kKS, false>
+                    : backend == kPlain ? (const void*)&k_step_mixed<kPlain, false>
+                    : backend == kFancy ? (const void*)&k_step_mixed<kFancy, false>
+                                        : (const void*)&k_step_mixed<kByte, false>;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, kTWG, 0) != hipSuccess || per_cu < 1) {
         (void)hipGetLastError();
@@ -977,25 +1105,36 @@ int step_grid(int backend, int n_cu) {
     return per_cu * n_cu;
 }
 
-// One step: start (roots, fills), expand/leaf segments in one mixed launch,
-// the late leaf passes (over levels the mixed launch wrote), up_rounds
-// (<= kUpRounds) upsweep rounds.  up_grid * 256 must cover
-// kMaxRoots and kMaxSegs (the roots and the outcomes are handled by the first
-// threads of the start kernel).
-// The step's start, mixed and (late) late launches for one backend and tiling.
+// One step: fetch, start (roots, fills), expand/leaf segments in one mixed
+// launch, the late leaf passes (over levels the mixed launch wrote), up_rounds
+// (<= kUpRounds) upsweep rounds, outcomes to the host.  up_grid * 256 must
+// cover kMaxRoots and kMaxSegs (the roots and the outcomes are handled by the
+// first threads of the start kernel).  A small step's fetch and start are one
+// launch, and so are its upsweeps and outcomes, as each of its kernels is a
+// launch's latency (4 to 5 us) and little else: a request at depth 4 on an idle
+// server, two steps, 95.8 -> 89.2 us.
 template <int B, bool F>
-static void launch_step_front(const SliderTables* tabs, const ZTables* zt, StepTable* t, uint4* tt, u64 mask, int grid,
-                              int up_grid, int late, hipStream_t s) {
-    hipLaunchKernelGGL(k_pre_step<B>, dim3(up_grid), dim3(256), 0, s, tabs, t, t->seg, tt, mask);
-    hipLaunchKernelGGL((k_step_mixed<B, kTTMixedWaves, F>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
-    if (late) hipLaunchKernelGGL((k_step_late<B, kTTLeafWaves>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
+static void launch_step_front(const SliderTables* tabs, const ZTables* zt, StepTable* t, const StepTable* h, uint4* tt,
+                              u64 mask, int grid, int up_grid, bool small, int late, hipStream_t s) {
+    if (small) {
+        hipLaunchKernelGGL(k_fetch_pre<B>, dim3(kSmallFetchGrid), dim3(256), 0, s, tabs, t, h, tt, mask);
+    } else {
+        hipLaunchKernelGGL(k_fetch_step, dim3(32), dim3(256), 0, s, t, h);
+        hipLaunchKernelGGL(k_pre_step<B>, dim3(up_grid), dim3(256), 0, s, tabs, t, t->seg, tt, mask);
+    }
+    hipLaunchKernelGGL((k_step_mixed<B, F>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
+    if (late) hipLaunchKernelGGL((k_step_late<B>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
 }
 
-hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt, StepTable* t, uint4* tt, u64 mask,
-                       int grid, int up_grid, int up_rounds, int fine, int late, hipStream_t s) {
+hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt, StepTable* t, StepTable* h, uint4* tt,
+                       u64 mask, int grid, int up_grid, int up_rounds, StepForm form, int late, u32 max_jobs,
+                       hipStream_t s) {
     if (up_grid * 256 < kMaxRoots || up_grid * 256 < kMaxSegs) return hipErrorInvalidValue;
+    static_assert(kSmallFetchGrid * 256 >= kMaxRoots && kSmallFetchGrid * 256 >= kMaxSegs, "one per thread");
     if (up_rounds < 0 || up_rounds > kUpRounds) return hipErrorInvalidValue;
-    using Front = void (*)(const SliderTables*, const ZTables*, StepTable*, uint4*, u64, int, int, int, hipStream_t);
+    using Front = void (*)(const SliderTables*, const ZTables*, StepTable*, const StepTable*, uint4*, u64, int, int,
+                           bool, int, hipStream_t);
+    const bool fine = form != kStepCoarse, small = form == kStepSmall;
     Front front;
     switch (backend) {
     case kKS: front = fine ? launch_step_front<kKS, true> : launch_step_front<kKS, false>; break;
@@ -1003,8 +1142,13 @@ hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt,
     case kFancy: front = fine ? launch_step_front<kFancy, true> : launch_step_front<kFancy, false>; break;
     default: front = fine ? launch_step_front<kByte, true> : launch_step_front<kByte, false>; break;
     }
-    front(tabs, zt, t, tt, mask, grid, up_grid, late, s);
-    for (int r = 0; r < up_rounds; r++) hipLaunchKernelGGL(k_up_step, dim3(up_grid), dim3(256), 0, s, t, tt, mask, r);
+    front(tabs, zt, t, h, tt, mask, grid, up_grid, small, late, s);
+    if (small) {
+        hipLaunchKernelGGL(k_up_post, dim3(1), dim3(kSmallWG), 0, s, t, h, tt, mask, up_rounds, max_jobs);
+    } else {
+        for (int r = 0; r < up_rounds; r++) hipLaunchKernelGGL(k_up_step, dim3(up_grid), dim3(256), 0, s, t, tt, mask, r);
+        hipLaunchKernelGGL(k_post_step, dim3(1), dim3(256), 0, s, t, h, max_jobs);
+    }
     return hipGetLastError();
 }
 
@@ -1183,7 +1327,6 @@ __global__ __launch_bounds__(64) void k_plan_leaf(TTPlanCtl* c, StepTable* t, in
     a.err = &t->out[0].err;
     a.stats = ttstats;
     t->seg[0] = a;
-    t->tile_prefix[1] = (u32)((cur.n + kTTP - 1) / kTTP);
     t->nseg = 1;
 }
 
@@ -1231,14 +1374,14 @@ static void plan_steps(const SliderTables* tabs, const ZTables* zt, TTPlanCtl* c
         // the write launch; at the last write level, when its planner chose to
         // fuse the leaf pass (StepTable::fuse_leaf), it leaves at once and the
         // fused launch runs the level instead
-        hipLaunchKernelGGL((k_step<B, kTTWaves, kWrite>), dim3(write_grid), dim3(kTWG), 0, s, tabs, zt, tab);
+        hipLaunchKernelGGL((k_step_write<B>), dim3(write_grid), dim3(kTWG), 0, s, tabs, zt, tab);
         if (L == r - 3)
-            hipLaunchKernelGGL((k_step_write_leaf<B, kTTMixedWaves>), dim3(leaf_grid), dim3(kTWG), 0, s, tabs, zt,
+            hipLaunchKernelGGL((k_step_write_leaf<B>), dim3(leaf_grid), dim3(kTWG), 0, s, tabs, zt,
                                tab);
     }
     // records the leaf level; the leaf launch is empty when the write fused it
     hipLaunchKernelGGL(k_plan_leaf, dim3(1), dim3(64), 0, s, ctl, tab, r - 2, ttstats);
-    hipLaunchKernelGGL((k_step<B, kTTLeafWaves, kLeaf>), dim3(leaf_grid), dim3(kTWG), 0, s, tabs, zt, tab);
+    hipLaunchKernelGGL((k_step_leaf<B>), dim3(leaf_grid), dim3(kTWG), 0, s, tabs, tab);
     for (int L = r - 3; L >= 0; L--) {
         hipLaunchKernelGGL(k_plan_up, dim3(1), dim3(64), 0, s, ctl, tab, L, ttstats);
         hipLaunchKernelGGL(k_up_step, dim3(up_grid), dim3(256), 0, s, tab, tt, mask, 0);
@@ -1265,16 +1408,22 @@ hipError_t capture_plan_pass(int backend, const SliderTables* tabs, const ZTable
 }
 
 // ---- launchers ---------------------------------------------------------------
-template <int M>
-static void* pick_mode(int backend) {
+static void* pick(int backend, int mode) {
+    if (mode == kLeaf) {
+        switch (backend) {
+        case kKS: return reinterpret_cast<void*>(&k_expand_tt_leaf<kKS>);
+        case kPlain: return reinterpret_cast<void*>(&k_expand_tt_leaf<kPlain>);
+        case kFancy: return reinterpret_cast<void*>(&k_expand_tt_leaf<kFancy>);
+        default: return reinterpret_cast<void*>(&k_expand_tt_leaf<kByte>);
+        }
+    }
     switch (backend) {
-    case kKS: return reinterpret_cast<void*>(&k_expand_tt<kKS, M>);
-    case kPlain: return reinterpret_cast<void*>(&k_expand_tt<kPlain, M>);
-    case kFancy: return reinterpret_cast<void*>(&k_expand_tt<kFancy, M>);
-    default: return reinterpret_cast<void*>(&k_expand_tt<kByte, M>);
+    case kKS: return reinterpret_cast<void*>(&k_expand_tt<kKS>);
+    case kPlain: return reinterpret_cast<void*>(&k_expand_tt<kPlain>);
+    case kFancy: return reinterpret_cast<void*>(&k_expand_tt<kFancy>);
+    default: return reinterpret_cast<void*>(&k_expand_tt<kByte>);
     }
 }
-static void* pick(int backend, int mode) { return mode == kLeaf ? pick_mode<kLeaf>(backend) : pick_mode<kWrite>(backend); }
 
 static int tt_bpc(void* f) {
     int per_cu = 0;
@@ -1290,11 +1439,16 @@ int expand_tt_leaf_bpc(int backend) { return tt_bpc(pick(backend, kLeaf)); }
 hipError_t launch_expand_tt(int backend, const SliderTables* tabs, const ZTables* zt, const TTArgs& a, int grid,
                             hipStream_t s) {
     if (!a.n_in) return hipSuccess;
+    TTArgs args = a;
+    if (a.mode == kLeaf) {  // the kernel tiles the level for its grid
+        if ((u32)grid > a.n_in) grid = (int)a.n_in;
+        void* kargs[] = {(void*)&tabs, (void*)&args};
+        return hipLaunchKernel(pick(backend, kLeaf), dim3(grid), dim3(kTWG), kargs, 0, s);
+    }
     const u32 tiles = (a.n_in + kTTP - 1) / kTTP;
     if ((u32)grid > tiles) grid = (int)tiles;
-    TTArgs args = a;
     void* kargs[] = {(void*)&tabs, (void*)&zt, (void*)&args};
-    return hipLaunchKernel(pick(backend, a.mode), dim3(grid), dim3(kTWG), kargs, 0, s);
+    return hipLaunchKernel(pick(backend, kWrite), dim3(grid), dim3(kTWG), kargs, 0, s);
 }
 
 hipError_t launch_roots_tt(int backend, const SliderTables* tabs, Board* roots, const u64* k1, const u64* k2, u32 n,

@@ -16,6 +16,8 @@ constexpr int kMinTTDepth = 3;
 // Parents per tile of the table kernels (a tile's move list is one LDS
 // window of 4096 entries); the serving step's tile prefix counts with it too.
 constexpr int kTTTileParents = 112;
+// Parents per tile of a leaf pass by sets (one per thread).
+constexpr int kTTLeafParents = 256;
 
 // In-level duplicate detection, at the moment a child is made (open
 // addressing, linear probing).  `key` is the child's second Zobrist key
@@ -90,6 +92,18 @@ constexpr int kMaxLate = 16;
 // this many parents (about 30 children each: one child per thread of a
 // workgroup), the fewest that still give every tile a workgroup of the launch.
 constexpr u32 kFineMinParents = 8;
+
+// Serving: a small step (at most these many write segments, upsweep segments
+// per round, upsweep items and 16-byte entries to clear) runs its upsweeps in
+// one workgroup and its clears in the kernel that fetches the table.  The
+// bounds keep either at a few passes of its workgroups (4 of 1024 items, 8 of
+// 8192 entries, about a microsecond each), below the launch that it saves.
+constexpr int kSmallSegs = 8;
+constexpr int kSmallUps = 64;
+constexpr u32 kSmallItems = 4096;
+constexpr u64 kSmallFill = 65536;
+constexpr int kSmallWG = 1024;
+constexpr int kSmallFetchGrid = 32;
 
 struct SegOut {
     u32 out_count;
@@ -233,19 +247,23 @@ hipError_t capture_plan_pass(int backend, const SliderTables* tabs, const ZTable
                              u64 mask, unsigned long long* ttstats, int r, int write_grid, int leaf_grid,
                              int up_grid, hipStream_t s);
 
-// Serving: the used part of the step table from coherent host memory `h`
-// into `d`; the step's outcomes from `d` back into `h`, then h->done = d->seq
-// once every outcome is visible to the host.
-hipError_t launch_fetch_step(StepTable* d, const StepTable* h, hipStream_t s);
-hipError_t launch_post_step(const StepTable* d, StepTable* h, u32 max_jobs, hipStream_t s);
 // *flag = v (host memory, system scope) once the stream's earlier work is done.
 hipError_t launch_post_flag(u32* flag, u32 v, hipStream_t s);
 int step_grid(int backend, int n_cu);       // workgroups of the serving step's mixed launch
 int step_max_bpc(int backend, int leaf);  // the planned pass's write (0) / leaf (1) step kernel
-// fine: the mixed launch tiles by StepTable::mix_tp parents, not kTTTileParents;
-// late: the late leaf launch is recorded (steps with StepTable::nlate > 0)
-hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt, StepTable* t, uint4* tt, u64 mask,
-                       int grid, int up_grid, int up_rounds, int fine, int late, hipStream_t s);
+// The serving step: the used part of the step table from coherent host memory
+// `h` into `t`, the step, its outcomes back into `h`, then h->done = t->seq
+// once every outcome is visible to the host.
+// late: the late leaf launch is recorded (steps with StepTable::nlate > 0).
+enum StepForm {
+    kStepCoarse,  // the mixed launch tiles by kTTTileParents parents
+    kStepFine,    // ... by StepTable::mix_tp
+    kStepSmall,   // fine, within the kSmall* bounds: fewer launches
+    kStepForms
+};
+hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt, StepTable* t, StepTable* h, uint4* tt,
+                       u64 mask, int grid, int up_grid, int up_rounds, StepForm form, int late, u32 max_jobs,
+                       hipStream_t s);
 int expand_tt_max_bpc(int backend);   // most resident workgroups per CU of the TT write-level kernel
 int expand_tt_leaf_bpc(int backend);  // the same for the TT leaf-level kernel
 hipError_t launch_expand_tt(int backend, const SliderTables* tabs, const ZTables* zt, const TTArgs& a, int grid,

@@ -135,3 +135,51 @@ def test_leaf_records_overflow(pg, leaf, engine):
         assert sound
         for i in sound:
             assert int(got[i]) == leaf.lc_perft2_moves(base[i:].ctypes.data), base[i]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("backend,graphs,dedup", [("ks", True, True), ("ks", False, True), ("ks", False, False),
+                                                  ("fancy", True, True), ("byte", False, True)])
+def test_table_leaf_level(pg, oracle, backend, graphs, dedup):
+    """leaf passes of the table search on either side of 32 parents a
+    workgroup, in planned passes (two launches, or the last write level and
+    its leaf pass in one) and level by level from the host"""
+    pos = pg.playouts(4321, 1500, 8, 60)
+    for n, d in ((1, 3), (40, 3), (701, 3), (20, 4), (900, 4), (1500, 4), (60, 5)):
+        want = oracle.perft_batch(pos[:n], d, nthreads=8)
+        eng = pg.Engine(backend=backend, arena_bytes=4 << 30, tt_bytes=1 << 28, zobrist_seed=7)
+        try:
+            eng.set_level_graphs(graphs)
+            eng.set_dedup(dedup)
+            assert np.array_equal(eng.perft_batch(pos[:n], d), want), (n, d)
+        finally:
+            eng.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tt_bytes", [0, 1 << 28])
+@pytest.mark.parametrize("jobs,n,dmax", [(1, 6, 4), (4, 30, 4), (64, 300, 4), (64, 200, 5)])
+def test_serving_step_forms(pg, oracle, tt_bytes, jobs, n, dmax):
+    """steps small enough for the fewer launches, finely tiled ones and large
+    ones, with leaf passes in the write's step and after it"""
+    pos = pg.playouts(99, n, 8, 60)
+    depth = [1 + (i * 7) % dmax for i in range(n)]
+    want = {}
+    for d in sorted(set(depth)):
+        sel = [i for i in range(n) if depth[i] == d]
+        want.update(zip(sel, oracle.perft_batch(np.ascontiguousarray(pos[sel]), d, nthreads=8)))
+    eng = pg.Engine(arena_bytes=4 << 30, tt_bytes=tt_bytes)
+    try:
+        for wait_each in (True, False):
+            eng.serve_start(max_jobs=jobs)
+            got = {}
+            for i in range(n):
+                eng.submit(pos[i], depth[i], i)
+                while wait_each and i not in got:
+                    got.update((r["tag"], r["nodes"]) for r in eng.poll())
+            while len(got) < n:
+                got.update((r["tag"], r["nodes"]) for r in eng.poll())
+            eng.serve_stop()
+            assert got == {i: int(w) for i, w in want.items()}
+    finally:
+        eng.close()
