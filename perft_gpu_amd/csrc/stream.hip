@@ -61,6 +61,9 @@ template <int MODE, bool SETS, int TP, int CAP, int WG, class MakeSl>
 __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const PersistArgs& p, int L,
                                              TileLds<TP, CAP, WG>& s, LeafLevelLds* sets) {
     PersistCtl* ctl = p.ctl;
+    // What the previous launches left, read in one go: a small level waits on
+    // each of these reads.
+    const u64 nl = ctl->totals[L], lo = ctl->lvl_off[L], nn = ctl->totals[L + 1];
     // an earlier level did not fit: nothing below it is counted (one read per
     // workgroup, so that the whole workgroup leaves together)
     if (threadIdx.x == 0) s.ok = ctl->err;
@@ -70,8 +73,8 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
     const u32* cur_r = p.root_ids;
     u64 n = p.n_roots, off = 0;
     if (L > 0) {
-        n = ctl->totals[L];
-        off = ctl->lvl_off[L];
+        n = nl;
+        off = lo;
         cur = reinterpret_cast<const Board*>(p.arena + off);
         cur_r = reinterpret_cast<const u32*>(p.arena + off + ((n * sizeof(Board) + 255) & ~255ULL));
         off += ((n * sizeof(Board) + 255) & ~255ULL) + ((n * sizeof(u32) + 255) & ~255ULL);
@@ -104,7 +107,6 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
         expand_level(sl, a, kLeaf, s);
         return;
     }
-    const u64 nn = ctl->totals[L + 1];
     const u64 bbytes = (nn * sizeof(Board) + 255) & ~255ULL, rbytes = (nn * sizeof(u32) + 255) & ~255ULL;
     if (nn > 0xFFFFFFFFull || off + bbytes + rbytes > p.arena_bytes) {
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&ctl->err, 2u);
