@@ -92,7 +92,7 @@ typedef struct pf_stats {
     uint64_t chunks;          /* depth-first chunk splits taken */
     uint64_t peak_arena_bytes;
     uint64_t tt_probes, tt_hits, tt_stores;  /* while serving: probes and hits since pf_serve_start */
-    double gpu_ms;            /* device time of expand kernels (HIP events) */
+    double gpu_ms;            /* device time of expand kernels (HIP events, or the device clock) */
     double last_expand_ms;    /* average duration of the last run's expand launches */
     uint64_t last_expand_launches;
     uint64_t dup_nodes;       /* nodes found to duplicate another node of their level (TT runs) */

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 
+#include "serve.h"
 #include "tables.h"
 
 namespace pf {
@@ -63,6 +64,12 @@ pf_status Engine::init(const pf_config& cfg) {
     PF_HIP(hipMalloc(&d_ctrl, 64 * sizeof(u32)));
     PF_HIP(hipMalloc(&d_total, 8 * sizeof(unsigned long long)));
     PF_HIP(hipHostMalloc(&h_pinned, 64 * sizeof(unsigned long long), hipHostMallocDefault));
+    PF_HIP(hipHostMalloc(&h_io, sizeof(StreamIO), hipHostMallocCoherent | hipHostMallocMapped));
+    PF_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&d_io), h_io, 0));
+    h_io->done = io_seq;
+    int khz = 0;
+    PF_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+    clock_khz = khz;
     PF_HIP(hipEventCreate(&ev0));
     PF_HIP(hipEventCreate(&ev1));
     PF_HIP(hipMalloc(&d_pctl, sizeof(PersistCtl)));
@@ -96,11 +103,12 @@ void Engine::destroy() {
     hipHostFree(h_pstat);
     d_plan = nullptr; d_ptab = nullptr; h_plan = nullptr; h_pstat = nullptr;
     hipHostFree(h_pinned);
+    hipHostFree(h_io);
     if (ev0) hipEventDestroy(ev0);
     if (ev1) hipEventDestroy(ev1);
     if (stream) hipStreamDestroy(stream);
     d_tab = nullptr; arena = nullptr; d_ctrl = nullptr; d_total = nullptr;
-    d_sums = nullptr; d_wsums = nullptr; h_pinned = nullptr; stream = nullptr; d_pctl = nullptr;
+    d_sums = nullptr; d_wsums = nullptr; h_pinned = nullptr; h_io = d_io = nullptr; stream = nullptr; d_pctl = nullptr;
 }
 
 pf_status Engine::ensure_sums(u64 n) {
@@ -280,8 +288,77 @@ pf_status Engine::perft_levels(const pf_pos48* pos, int n, int d, u64* out) {
     return PF_OK;
 }
 
+// The post kernel writes io->done once everything the host needs has reached
+// it, some microseconds before the stream's completion would wake a waiting
+// thread, so the caller watches the word.  Work still running after kSpinS is
+// waited for by hipStreamSynchronize, which also reports a failed launch.
+pf_status Engine::wait_small() {
+    constexpr double kSpinS = 0.001;
+    const double t0 = now_s();
+    while (__atomic_load_n(&h_io->done, __ATOMIC_ACQUIRE) != io_seq) {
+        if (now_s() - t0 > kSpinS) {
+            if (hipStreamSynchronize(stream) != hipSuccess ||
+                __atomic_load_n(&h_io->done, __ATOMIC_ACQUIRE) != io_seq)
+                return PF_EDEVICE;
+            break;
+        }
+        __builtin_ia32_pause();
+    }
+    return h_io->err & 2 ? PF_ENOMEM : h_io->err ? PF_EDEVICE : PF_OK;
+}
+
+void Engine::add_small_time() {
+    if (!timing) return;
+    const double ms = (double)(h_io->t1 - h_io->t0) / clock_khz;
+    st.gpu_ms += ms;
+    st.last_expand_ms = ms;
+    st.last_expand_launches = 1;
+}
+
+// A batch of at most kStreamSmall roots (kernels.h).
+pf_status Engine::perft_stream_small(const pf_pos48* pos, int n, int d, u64* out, bool dev_in, bool dev_out) {
+    PF_HIP(hipSetDevice(device));
+    pf_status s = ensure_sums((u64)n);
+    if (s != PF_OK) return s;
+    char* mark = arena + arena_top;
+    PersistArgs p;
+    p.roots = reinterpret_cast<Board*>(alloc((u64)n * sizeof(Board)));
+    p.root_ids = reinterpret_cast<u32*>(alloc((u64)n * sizeof(u32)));
+    if (!p.roots || !p.root_ids) {
+        release(mark);
+        return PF_ENOMEM;
+    }
+    p.n_roots = (u32)n;
+    p.depth = d;
+    p.arena = arena + arena_top;
+    p.arena_bytes = arena_bytes - arena_top;
+    p.ctl = d_pctl;
+    p.sums = d_sums;
+    release(mark);  // (nothing else takes arena memory before the pass has ended)
+    if (!dev_in) memcpy(h_io->pos, pos, (size_t)n * sizeof(pf_pos48));
+    const int var[2] = {tune[backend].s_leaf, tune[backend].s_write};
+    io_seq++;
+    if (launch_stream_small(backend, DevTables{d_tab}, p, dev_in ? pos : d_io->pos, sgrid[backend], var, stream) !=
+            hipSuccess ||
+        launch_stream_post(p, dev_out ? reinterpret_cast<unsigned long long*>(out) : nullptr, d_io, io_seq, stream) !=
+            hipSuccess) {
+        (void)hipStreamSynchronize(stream);  // what was launched may still read the positions
+        return PF_EDEVICE;
+    }
+    st.kernel_launches += (u64)d + 1;  // the begin and the post kernel and d - 1 levels
+    st.levels_run += (u64)(d - 1);
+    s = wait_small();
+    if (s != PF_OK) return s;
+    // device results: complete for any stream or engine once the stream is
+    if (dev_out && hipStreamSynchronize(stream) != hipSuccess) return PF_EDEVICE;
+    add_small_time();
+    if (!dev_out) memcpy(out, h_io->sums, (size_t)n * 8);
+    return PF_OK;
+}
+
 pf_status Engine::perft_stream(const pf_pos48* pos, int n, int d, u64* out, bool dev_in, bool dev_out) {
     if (n <= 0) return PF_OK;
+    if (d >= 1 && n <= (int)kStreamSmall) return perft_stream_small(pos, n, d, out, dev_in, dev_out);
     if (d <= 1) {
         if (dev_in || dev_out) return PF_EINVAL;  // callers stage shallow device batches themselves
         return perft_levels(pos, n, d, out);

@@ -33,6 +33,10 @@ struct Engine {
     unsigned long long* d_wsums = nullptr;   // per-root sums of expand-and-write launches
     u64 sums_cap = 0;
     unsigned long long* h_pinned = nullptr;  // small pinned readback buffer
+    StreamIO* h_io = nullptr;   // small stream-ordered batches: positions in, outcome back
+    StreamIO* d_io = nullptr;   // h_io as the device addresses it
+    u32 io_seq = 0;             // number of the last batch
+    double clock_khz = 0;       // of the device clock in StreamIO
 
     int grid[4][2] = {};        // level-loop launches on large levels (wide tile, five waves per SIMD)
     int grid_small[4][2] = {};  // the same on small levels (256 x 8192 tile)
@@ -128,6 +132,10 @@ struct Engine {
     pf_status expand(int mode, const Board* in, const u32* in_root, u64 n_in, Board* out, u32* out_root,
                      u64 out_cap, unsigned long long* sums, u64* next_total);
     pf_status range_count(const Board* b, u64 n, u64* total);
+    // Waits for the batch that launch_stream_post posts as io_seq; adds its time.
+    pf_status wait_small();
+    void add_small_time();
+    pf_status perft_stream_small(const pf_pos48* pos, int n, int depth, u64* out, bool dev_in, bool dev_out);
     pf_status upload_roots(const pf_pos48* pos, int n, Board** roots, u32** rid, bool dev_in = false);
     pf_status descend(const Board* lvl, const u32* rts, u64 n, u64 n_next, int L);
     bool alloc_tlevel(u64 n, TLevel* lv);

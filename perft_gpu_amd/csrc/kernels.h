@@ -66,6 +66,7 @@ struct PersistCtl {
     u32 pad[3];
     unsigned long long totals[20];  // totals[L] = number of nodes of level L
     unsigned long long lvl_off[20];  // stream-ordered form: arena offset of level L
+    unsigned long long t0;           // stream-ordered form, small batches: device clock at its begin kernel
 };
 struct PersistArgs {
     Board* roots;
@@ -96,5 +97,29 @@ constexpr int kStreamWriteDefault = 3;   // 256 x 4096 tile, no waves target
 int stream_grid(int backend, int mode, int variant, int n_cu);
 hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a, const int grid[2],
                          const int variant[2], hipStream_t s);
+
+// A batch of at most kStreamSmall roots: `pos` (reference layout; coherent
+// host or device memory) is converted, counted and its control block cleared
+// by one launch of one workgroup in front of the levels (depth >= 1), and its
+// outcome posted to the host's StreamIO by one behind them, in place of three
+// clears, two or three copies and their waits.  One position (whose levels
+// the host sized one by one before) at depth 3 133 -> 35 us and at depth 5 230
+// -> 81, a divide at depth 5 159 -> 87, 37 positions at perft 4 179 -> 104, 100
+// in device memory 141 -> 128.  1024 is one workgroup's threads: the begin of
+// more roots would wait on passes of a single CU.
+constexpr u32 kStreamSmall = 1024;
+struct StreamIO {  // coherent host memory
+    u32 done;      // the call's number, written after the rest
+    u32 err;       // PersistCtl::err
+    unsigned long long t0, t1;  // device clock at the begin and the post kernel
+    unsigned long long sums[kStreamSmall];
+    pf_pos48 pos[kStreamSmall];
+};
+// The levels as above, behind the begin kernel.
+hipError_t launch_stream_small(int backend, const DevTables& dt, const PersistArgs& a, const pf_pos48* pos,
+                               const int grid[2], const int variant[2], hipStream_t s);
+// The sums to dev_out (null: io->sums; a.sums: they are there), then the rest
+// of *io, then io->done = seq.
+hipError_t launch_stream_post(const PersistArgs& a, unsigned long long* dev_out, StreamIO* io, u32 seq, hipStream_t s);
 
 }  // namespace pf

@@ -41,8 +41,9 @@ static hipError_t scratch_address(int device, void** out) {
     return hipSuccess;
 }
 
-// Clears the control block and the caller's counts (a fill kernel, not a
-// memset, so that the whole call can be captured in a graph).
+// Clears the control block and the caller's counts where the begin kernel of a
+// small batch does not (a fill kernel, not a memset, so that the whole call can
+// be captured in a graph).
 __global__ __launch_bounds__(256) void k_noalloc_clear(PersistCtl* ctl, unsigned long long* out, u32 n,
                                                        unsigned long long fill) {
     const u32 i = blockIdx.x * 256 + threadIdx.x;
@@ -69,13 +70,6 @@ pf_status Engine::perft_noalloc(const pf_pos48* dpos, int n, int d, u64* dout) {
     u32* rid = reinterpret_cast<u32*>(s + ctl_b + roots_b);
     unsigned long long* out = reinterpret_cast<unsigned long long*>(dout);
 
-    const u32 words = (u32)(sizeof(PersistCtl) / 4);
-    const u32 clear_n = std::max<u32>((u32)n, words);
-    hipLaunchKernelGGL(k_noalloc_clear, dim3((clear_n + 255) / 256), dim3(256), 0, stream, ctl, out, (u32)n,
-                       d <= 0 ? 1ULL : 0ULL);
-    if (hipGetLastError() != hipSuccess) return PF_EDEVICE;
-    if (d <= 0) return hipStreamSynchronize(stream) == hipSuccess ? PF_OK : PF_EDEVICE;
-    if (launch_pos_to_board(dpos, (u32)n, roots, rid, stream) != hipSuccess) return PF_EDEVICE;
     PersistArgs p;
     p.roots = roots;
     p.root_ids = rid;
@@ -85,27 +79,41 @@ pf_status Engine::perft_noalloc(const pf_pos48* dpos, int n, int d, u64* dout) {
     p.arena_bytes = kScratchBytes - (ctl_b + roots_b + rid_b);
     p.ctl = ctl;
     p.sums = out;
-    if (timing && hipEventRecord(ev0, stream) != hipSuccess) return PF_EDEVICE;
+    const bool small = n <= (int)kStreamSmall && d >= 1;
     const int var[2] = {tune[backend].s_leaf, tune[backend].s_write};
-    if (launch_stream(backend, DevTables{d_tab}, p, sgrid[backend], var, stream) != hipSuccess) return PF_EDEVICE;
-    if (timing && hipEventRecord(ev1, stream) != hipSuccess) return PF_EDEVICE;
-    st.kernel_launches += (u64)d + 2;  // clear, conversion, the root count and d - 1 levels
+    if (small) {
+        if (launch_stream_small(backend, DevTables{d_tab}, p, dpos, sgrid[backend], var, stream) != hipSuccess)
+            return PF_EDEVICE;
+    } else {
+        const u32 words = (u32)(sizeof(PersistCtl) / 4);
+        const u32 clear_n = std::max<u32>((u32)n, words);
+        hipLaunchKernelGGL(k_noalloc_clear, dim3((clear_n + 255) / 256), dim3(256), 0, stream, ctl, out, (u32)n,
+                           d <= 0 ? 1ULL : 0ULL);
+        if (hipGetLastError() != hipSuccess) return PF_EDEVICE;
+        if (d <= 0) return hipStreamSynchronize(stream) == hipSuccess ? PF_OK : PF_EDEVICE;
+        if (launch_pos_to_board(dpos, (u32)n, roots, rid, stream) != hipSuccess) return PF_EDEVICE;
+        if (timing && hipEventRecord(ev0, stream) != hipSuccess) return PF_EDEVICE;
+        if (launch_stream(backend, DevTables{d_tab}, p, sgrid[backend], var, stream) != hipSuccess) return PF_EDEVICE;
+        if (timing && hipEventRecord(ev1, stream) != hipSuccess) return PF_EDEVICE;
+    }
+    st.kernel_launches += (u64)d + (small ? 1 : 3);  // the d - 1 levels and the kernels around them
     st.levels_run += (u64)(d - 1);
-    // the overflow flag comes back through the pinned buffer allocated at init
-    if (hipMemcpyAsync(h_pinned, &ctl->err, sizeof(u32), hipMemcpyDeviceToHost, stream) != hipSuccess ||
-        hipStreamSynchronize(stream) != hipSuccess)
-        return PF_EDEVICE;
-    if (timing) {
+    // the overflow flag comes back through the host words allocated at init
+    io_seq++;
+    if (launch_stream_post(p, out, d_io, io_seq, stream) != hipSuccess) return PF_EDEVICE;
+    const pf_status s2 = wait_small();
+    // (the counts are complete for any stream or engine once the stream is)
+    if (hipStreamSynchronize(stream) != hipSuccess) return PF_EDEVICE;
+    if (small) {
+        add_small_time();
+    } else if (timing) {
         float ms = 0;
         hipEventElapsedTime(&ms, ev0, ev1);
         st.gpu_ms += ms;
         st.last_expand_ms = ms;
         st.last_expand_launches = 1;
     }
-    const u32 err = *reinterpret_cast<const u32*>(h_pinned);
-    if (err & 2) return PF_ENOMEM;  // a level did not fit the scratch array
-    if (err) return PF_EDEVICE;
-    return PF_OK;
+    return s2;
 }
 
 }  // namespace pf

@@ -23,6 +23,7 @@
 // VGPRs, no spills) of the same source is exact and as fast.
 #include <hip/hip_runtime.h>
 
+#include "convert.h"
 #include "level_dev.h"
 
 namespace pf {
@@ -52,6 +53,48 @@ __global__ __launch_bounds__(kWG) void k_stream_roots(const SliderTables* tabs, 
     }
     c = wave_sum64(c);
     if ((threadIdx.x & 63) == 0 && c) atomicAdd(&p.ctl->totals[1], c);
+}
+
+// Begin of a small batch: one workgroup of a thread per root.
+template <int B>
+__global__ __launch_bounds__(kStreamSmall) void k_stream_begin(const SliderTables* tabs, PersistArgs p,
+                                                               const pf_pos48* __restrict__ pos) {
+    __shared__ unsigned long long red[kStreamSmall / 64];
+    constexpr u32 kWords = sizeof(PersistCtl) / 4;
+    const u32 i = threadIdx.x;
+    const unsigned long long t0 = wall_clock64();
+    unsigned long long c = 0;
+    if (i < p.n_roots) {
+        const Board b = to_board(pos[i]);
+        c = count_moves(b, SlOf<B>::make(tabs));
+        p.roots[i] = with_count(b, (u32)c);
+        p.root_ids[i] = i;
+        p.sums[i] = p.depth == 1 ? c : 0;
+    }
+    for (u32 w = i; w < kWords; w += blockDim.x) reinterpret_cast<u32*>(p.ctl)[w] = 0;
+    c = wave_sum64(c);
+    if ((i & 63) == 0) red[i >> 6] = c;
+    __syncthreads();  // (the words are cleared before two of them are set)
+    if (i == 0) {
+        unsigned long long t = 0;
+        for (u32 w = 0; w < blockDim.x / 64; w++) t += red[w];
+        p.ctl->totals[1] = t;
+        p.ctl->t0 = t0;
+    }
+}
+
+__global__ __launch_bounds__(kWG) void k_stream_post(const PersistCtl* ctl, const unsigned long long* sums, u32 n,
+                                                     unsigned long long* out, StreamIO* io, u32 seq) {
+    if (threadIdx.x == 0) {
+        io->err = ctl->err;
+        io->t0 = ctl->t0;
+        io->t1 = wall_clock64();
+    }
+    for (u32 i = threadIdx.x; i < n; i += blockDim.x) out[i] = sums[i];
+    __threadfence_system();  // this thread's writes reach the host before the barrier ...
+    __syncthreads();
+    if (threadIdx.x == 0)    // ... and so before done
+        __hip_atomic_store(&io->done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One level for one workgroup of the launch.  `make_sl` builds the slider
@@ -196,16 +239,10 @@ int stream_grid(int backend, int mode, int variant, int n_cu) {
                          stream_dyn(backend, variant)) * n_cu;
 }
 
-hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a, const int grid[2],
-                         const int variant[2], hipStream_t s) {
+// Levels 0..depth-2.
+static hipError_t launch_levels(int backend, const SliderTables* t, const PersistArgs& a, const int grid[2],
+                                const int variant[2], hipStream_t s) {
     PersistArgs args = a;
-    const SliderTables* t = dt.t;
-    {
-        void* kargs[] = {(void*)&t, (void*)&args};
-        const hipError_t e = hipLaunchKernel(pick_stream_roots(backend), dim3((a.n_roots + kWG - 1) / kWG), dim3(kWG),
-                                             kargs, 0, s);
-        if (e != hipSuccess) return e;
-    }
     for (int L = 0; L <= a.depth - 2; L++) {
         const int mode = (L == a.depth - 2) ? kLeaf : kWrite;
         void* kargs[] = {(void*)&t, (void*)&args, (void*)&L};
@@ -217,6 +254,38 @@ hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a,
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a, const int grid[2],
+                         const int variant[2], hipStream_t s) {
+    PersistArgs args = a;
+    const SliderTables* t = dt.t;
+    void* kargs[] = {(void*)&t, (void*)&args};
+    const hipError_t e = hipLaunchKernel(pick_stream_roots(backend), dim3((a.n_roots + kWG - 1) / kWG), dim3(kWG),
+                                         kargs, 0, s);
+    return e != hipSuccess ? e : launch_levels(backend, t, a, grid, variant, s);
+}
+
+hipError_t launch_stream_small(int backend, const DevTables& dt, const PersistArgs& a, const pf_pos48* pos,
+                               const int grid[2], const int variant[2], hipStream_t s) {
+    if (a.n_roots > kStreamSmall) return hipErrorInvalidValue;
+    const dim3 wg((a.n_roots + 63) / 64 * 64);
+    switch (backend) {
+    case kKS: hipLaunchKernelGGL(k_stream_begin<kKS>, dim3(1), wg, 0, s, dt.t, a, pos); break;
+    case kPlain: hipLaunchKernelGGL(k_stream_begin<kPlain>, dim3(1), wg, 0, s, dt.t, a, pos); break;
+    case kFancy: hipLaunchKernelGGL(k_stream_begin<kFancy>, dim3(1), wg, 0, s, dt.t, a, pos); break;
+    default: hipLaunchKernelGGL(k_stream_begin<kByte>, dim3(1), wg, 0, s, dt.t, a, pos); break;
+    }
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : launch_levels(backend, dt.t, a, grid, variant, s);
+}
+
+hipError_t launch_stream_post(const PersistArgs& a, unsigned long long* dev_out, StreamIO* io, u32 seq, hipStream_t s) {
+    const u32 n = dev_out == a.sums ? 0u : a.n_roots;  // counts to move
+    if (!dev_out && n > kStreamSmall) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_stream_post, dim3(1), dim3(n > 64 ? kWG : 64), 0, s, a.ctl, a.sums, n,
+                       dev_out ? dev_out : io->sums, io, seq);
+    return hipGetLastError();
 }
 
 }  // namespace pf
