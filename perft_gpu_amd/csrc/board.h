@@ -74,6 +74,14 @@ PF_HD u32 popc_add32(u32 x, u32 n) {
 #endif
     return n;
 }
+// Product of two numbers below 2^24: one full-rate instruction.
+PF_HD u32 mul24(u32 a, u32 b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __umul24(a, b);
+#else
+    return a * b;
+#endif
+}
 PF_HD int ctz(u64 x) { return __builtin_ctzll(x); }
 PF_HD u64 bit(int s) { return 1ULL << s; }
 PF_HD u64 flip(u64 x) { return __builtin_bswap64(x); }  // vertical mirror

@@ -77,13 +77,14 @@ struct LeafRecIter {
 };
 PF_HD u32 leaf_rec_moves(u64 to, u32 meta) {
     const u32 n = (u32)popc(to);
-    return ((meta >> 6) & 7) == 1 ? n + 3 * (u32)popc(to & kRank8) : n;
+    return ((meta >> 6) & 7) == 1 ? n + mul24((u32)popc(to & kRank8), 3) : n;
 }
 
 // P, bit-sliced in five digits.  On empty squares and on ours it is at most
 // 28: a line holds at most two of the opponent's rays through a square, which
 // see at most six squares beyond it, and pawns count at most four.  Captured
-// pieces can reach more; their squares are noted in `over`.
+// pieces can reach more; their squares are noted in `over`.  Few of ours reach
+// 16; their moves are handed out.
 struct LeafPlanes {
     u64 p[5], over;
     // t0 + 2 t1 + 4 t2 + 8 t3 on the squares of m, and 1 for every square of c
@@ -119,8 +120,8 @@ struct LeafPlanes {
         c &= p[i];
         p[i] = n;
     }
-    PF_HD u32 sum(u64 s) const {  // of P over the squares of s
-        u32 n = popc_add(s & p[4], 0);
+    PF_HD u32 sum(u64 s) const { return sum_from(s, popc_add(s & p[4], 0)); }  // of P over the squares of s
+    PF_HD u32 sum_from(u64 s, u32 n = 0) const {  // the same where no square of s reaches 16
 #pragma unroll
         for (int i = 3; i >= 0; i--) n = popc_add(s & p[i], n + n);
         return n;
@@ -380,7 +381,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
         const u64 f1 = push >> 8, p1 = f1 & empty, d1 = (p1 & kRank6) >> 8, p2 = d1 & empty;
         const u64 aSE = (cSE >> 7) & kNotA, aSW = (cSW >> 9) & kNotH, hSE = aSE & us, hSW = aSW & us;
         base = popc_add(hSE, popc_add(hSW, popc_add(p1 | p2, base)));  // the two kinds of push never share a target
-        base += 3 * popc_add32((u32)(p1 & kRank1), popc_add32((u32)(hSE & kRank1), popc_add32((u32)(hSW & kRank1), 0)));
+        base += mul24(popc_add32((u32)(p1 & kRank1), popc_add32((u32)(hSE & kRank1), popc_add32((u32)(hSW & kRank1), 0))), 3);
         pl.add2(or3(p1 | p2, f1 & us, p1 << 8), or3(p2 << 8, d1 & us, p2 << 16) | and3(f1 & kRank6, us, empty << 8));
         pl.add2(~aSE, ~aSW);
         pl.add2(hSE << 7, hSW << 9);
@@ -394,7 +395,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
         }
         const u64 edge = kRank1 & or3(f1, aSE, aSW);  // replies that promote
         zoneFrom = or3(zoneFrom, b.knights & knight_fill(za), p.pawns & pawn_from(za)) | (p.K & king_fill(za));
-        hardFrom |= edge;
+        hardFrom = or3(hardFrom, edge, pl.p[4]);
         if (generic) hardFrom = ~0ULL;
         hardTo = or3(hardTo, edge, pl.over) | (them & (king_fill(eK) | (tP & 0xFF00ULL)));
     }
@@ -410,12 +411,15 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
     const u64 att = or3(leaper_threats(b, pi), thr, beyond);  // where our king may not go
     const int rights = st_rights(b), ksq = pi.ksq;
     const u64 own = us & ~hardFrom;
-    u32 total = 0;
+    u32 total = 0, nOk = 0, nS = 0, nCap = 0;  // moves summed here; of those with `kings`, of captures
     // The moves of `t` (meta as in a record) of which those in `ok` need only
     // conditions on the opponent's king, and those in `s` none; the P of the
     // from squares of `ok` sum to fsum.
     auto take = [&](u64 t, u64 ok, u64 s, u32 fsum, u32 meta) {
-        total += popc_add(ok, 0) * base + popc_add(s, 0) * kings + popc_add(ok & them, 0) * cap + fsum - pl.sum(ok);
+        nOk = popc_add(ok, nOk);
+        nS = popc_add(s, nS);
+        nCap = popc_add(ok & them, nCap);
+        total += fsum - pl.sum(ok);
         emit(ok & ~s, t & ~ok, meta);
     };
     const bool check = pi.checkers != 0, dbl = (pi.checkers & (pi.checkers - 1)) != 0;
@@ -427,7 +431,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
         if (K & before7) ok &= ~(before7 & ((K << 8) | (K >> 8)));
         if (K & (or3(line[0], line[1], line[2]) | line[3])) ok = 0;
         const u64 s = (K & zoneFrom) ? 0 : ok & ~zoneTo & ~king_fill(zf);
-        take(t, ok, s, popc_add(ok, 0) * pl.sum(K), (u32)ksq);
+        take(t, ok, s, mul24(popc_add(ok, 0), pl.sum_from(K)), (u32)ksq);
     }
     const u64 tgt = dbl ? 0 : check ? (pi.checkers | pi.block) : ~us;
     const u64 free = ~pi.pinned;
@@ -437,7 +441,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
             const u64 sb = n & (0 - n), t = knight_fill(sb) & tgt;
             const int sq = ctz(n);
             const u64 ok = (sb & own) ? t & ~hard : 0, s = (sb & zoneFrom) ? 0 : ok & ~zone;
-            take(t, ok, s, popc_add(ok, 0) * pl.sum(sb), (u32)sq);
+            take(t, ok, s, mul24(popc_add(ok, 0), pl.sum_from(sb)), (u32)sq);
         }
     }
     // sliders, by kind; none of a line is `ok` if an opponent's slider sees the
@@ -466,7 +470,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
                 t &= (kf & sb) ? kf : (kr & sb) ? kr : (kd & sb) ? kd : anti_of(ksq);
             }
             const u64 ok = (sb & own) ? t & ~bad : 0, s = (sb & zoneFrom) ? 0 : ok & ~zone;
-            u32 f = popc_add(ok, 0) * pl.sum(sb);
+            u32 f = mul24(popc_add(ok, 0), pl.sum_from(sb));
             if (diag.value)  // a captured pawn's capture of ours is not lost twice
                 f = popc_add(ok & ((((sb << 9) & kNotA) & cSW) | (((sb << 7) & kNotH) & cSE)), f);
             take(t, ok, s, f, (u32)sq);
@@ -487,26 +491,26 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
             // a rook behind the pawn gains one square; a pawn of theirs two ranks
             // ahead loses its push and gains no double one
             const u64 t = q1 & tgt, ok = t & (own << 8) & ~hard;
-            const u32 f = popc_add(ok & (north << 8), pl.sum(ok >> 8)) - popc_add(and3(ok, before7, before7 << 8), 0);
+            const u32 f = popc_add(ok & (north << 8), pl.sum_from(ok >> 8)) - popc_add(and3(ok, before7, before7 << 8), 0);
             take(t, ok, ok & (calm << 8) & ~zone, f, 8u | kLeafPawn);
         }
         {
             const u64 t = (((check ? (q1 & ~tgt) : q1) & kRank3) << 8) & empty & tgt;
             const u64 ok = t & (own << 16) & ~(hard | ((u64)(beside >> 16) << 24));
             const u32 o4 = (u32)(ok >> 24), ep = popc_add32(o4 & beside, popc_add32(o4 & (beside >> 8), 0));
-            const u32 f = 2 * popc_add(ok & (north << 16), 0) + ep + pl.sum(ok >> 16);
+            const u32 f = 2 * popc_add(ok & (north << 16), 0) + ep + pl.sum_from(ok >> 16);
             take(t, ok, ok & (calm << 16) & ~zone, f, 16u | kLeafDouble);
         }
         // a captured pawn's capture of ours is not lost twice
         {
             const u64 t = ((or_and(Pf, pin, diag_of(ksq)) << 9) & kNotA) & them & tgt;
             const u64 ok = t & ((own & ~(line[2] | line[0])) << 9) & ~hard;
-            take(t, ok, ok & (calm << 9) & ~zone, popc_add(ok & cSW, pl.sum(ok >> 9)), 9u | kLeafPawn);
+            take(t, ok, ok & (calm << 9) & ~zone, popc_add(ok & cSW, pl.sum_from(ok >> 9)), 9u | kLeafPawn);
         }
         {
             const u64 t = ((or_and(Pf, pin, anti_of(ksq)) << 7) & kNotH) & them & tgt;
             const u64 ok = t & ((own & ~(line[3] | line[0])) << 7) & ~hard;
-            take(t, ok, ok & (calm << 7) & ~zone, popc_add(ok & cSE, pl.sum(ok >> 7)), 7u | kLeafPawn);
+            take(t, ok, ok & (calm << 7) & ~zone, popc_add(ok & cSE, pl.sum_from(ok >> 7)), 7u | kLeafPawn);
         }
     }
     {
@@ -536,7 +540,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
             emit(0, ok ? T : 0, (u32)(s ? ctz(s) : 0) | kLeafEP);
         }
     }
-    return total;
+    return total + nOk * base + nS * kings + nCap * cap;
 }
 
 }  // namespace pf

@@ -53,13 +53,15 @@ struct LeafEmit {
         more = more || ek + ef > (u32)N;
         if (more) return;
         if (k) {
-            const u32 at = ck + below(mk);
+            u32 at = ck + below(mk);
             pool->to[at] = k;
+            pin(at);  // (else meta's address is made from to's by a 64-bit multiply)
             pool->meta[at] = (u16)(meta | tag);
         }
         if (f) {
-            const u32 at = N - 1 - cf - below(mf);
+            u32 at = N - 1 - cf - below(mf);
             pool->to[at] = f;
+            pin(at);
             pool->meta[at] = (u16)(meta | tag);
         }
         nk = ek;
@@ -78,7 +80,11 @@ __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u
     const u32 lane = tid & 63, wid = uniform(tid >> 6);
     const LeafPool<N>& pool = s.pool[wid];
     u32 cnt = 0;
-    for (u32 r = r0 + lane; r < r1; r += 64) cnt += leaf_rec_moves(pool.to[r], pool.meta[r]);
+    for (u32 r = r0 + lane; r < r1; r += 64) {
+        u32 q = r;
+        pin(q);  // (as in LeafEmit)
+        cnt += leaf_rec_moves(pool.to[r], pool.meta[q]);
+    }
     const u32 incl = wave_incl_scan(cnt);
     if (lane == 63) s.wtot[wid] = incl;
     __syncthreads();
@@ -92,7 +98,9 @@ __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u
     for (u32 w0 = 0; w0 < tot; w0 += CAP) {
         u32 pos = woff + incl - cnt - w0;  // of the lane's next move, wrapping below the window
         for (u32 r = r0 + lane; r < r1; r += 64) {
-            const u32 meta = pool.meta[r], tag = ((meta >> kLeafMetaBits) | (wid << 6)) << 16;
+            u32 q = r;
+            pin(q);
+            const u32 meta = pool.meta[q], tag = ((meta >> kLeafMetaBits) | (wid << 6)) << 16;
             LeafRecIter it{pool.to[r], meta, 0};
             while (!it.done()) {
                 const u32 m = it.next();
@@ -104,8 +112,9 @@ __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u
         const u32 m = min((u32)CAP, tot - w0);
         for (u32 j = tid; j < m; j += WG) {
             const u32 x = s.mv[j], par = x >> 16;
-            const u32 c = KING ? leaf_king_replies(s.b[par], x & 0xFFFFu)
-                               : count_moves(make_move(s.b[par], x & 0xFFFFu), sl);
+            const Board& b = *reinterpret_cast<const Board*>(reinterpret_cast<const char*>(s.b) +
+                                                             mul24(par, sizeof(Board)));
+            const u32 c = KING ? leaf_king_replies(b, x & 0xFFFFu) : count_moves(make_move(b, x & 0xFFFFu), sl);
             atomicAdd(&s.sum[par], c);
         }
         __syncthreads();

@@ -292,7 +292,7 @@ PF_HD u32 count_pawns_knights(const Board& b, const PosInfo& pi, const CountMask
         u32 promo = popc_add32((u32)(cr >> 32) & kR8, 0u);
         promo = popc_add32((u32)(cl >> 32) & kR8, promo);
         promo = popc_add32((u32)((p1 & safe) >> 32) & kR8, promo);
-        n += 3 * promo;
+        n += mul24(promo, 3);
     }
     // en passant (MoveGeneratorBitboard.h:3058-3107; in check :2873-2890)
     const int ep = st_ep(b);
