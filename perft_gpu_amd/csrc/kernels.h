@@ -27,6 +27,7 @@ struct LevelArgs {
     u32* err;            // set non-zero on capacity overflow
     u32 tile_parents;    // parents per tile, at most the shape's (0: the shape's); a small level
                          // uses fewer, so that it spreads over more workgroups
+    bool uncounted = false;  // the children's moves are not counted (no total, no root_sums)
 };
 
 // Parents per tile for a level of n parents on `grid` workgroups of a shape
@@ -42,6 +43,7 @@ PF_HD u32 level_tile_parents(u64 n, u64 grid, u32 tp_max) {
 
 // A leaf level runs by sets (leaf.h) from this many parents per workgroup.
 constexpr u32 kLeafSetsMinParents = 32;
+constexpr u32 kLeafSetsTile = 256;  // its parents per tile
 
 enum ExpandMode : int { kLeaf = 0, kWrite = 1 };
 
@@ -77,6 +79,7 @@ struct PersistArgs {
     u64 arena_bytes;
     PersistCtl* ctl;
     unsigned long long* sums;
+    u32 leaf_grid = 0;  // stream-ordered form: workgroups of a leaf level that runs by sets
 };
 // Tile-shape variants of the persistent kernel (kernels.hip, PCfg) and the
 // most workgroups per CU that can be resident for one of them.

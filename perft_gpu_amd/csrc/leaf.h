@@ -280,9 +280,10 @@ PF_HD u32 leaf_king_replies(const Board& b, u32 m) {
 // opponent's replies; emit(king, full, meta) receives the others: records of
 // which only the replies of the opponent's king are missing, and of which all
 // are (either set may be empty).  On the GPU all lanes of a wave call it and
-// emit together; a lane without a position passes an empty board.
+// emit together; a lane without a position passes an empty board.  `summed`
+// (when not null) receives the number of moves not handed out in full.
 template <class SL, class Emit>
-PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
+PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit, u32* summed = nullptr) {
     // stage 1: pins of the opponent, squares each side attacks
     u64 pinT, thr, hardFrom, hardTo, za, zf, kR, kB, cast = 0;
     u32 base, kings, generic;  // replies but the king's; the king's
@@ -540,6 +541,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit) {
             emit(0, ok ? T : 0, (u32)(s ? ctz(s) : 0) | kLeafEP);
         }
     }
+    if (summed) *summed = nOk;
     return total + nOk * base + nS * kings + nCap * cap;
 }
 

@@ -72,9 +72,10 @@ struct LeafEmit {
 
 // Makes and counts the moves of the waves' records [r0, r1) (KING: only the
 // replies of the opponent's king are counted), adding to the parents' sums.
-// Ends with a barrier behind the last use of every LDS array.
+// Ends with a barrier behind the last use of every LDS array; returns the
+// number of moves.
 template <bool KING, class SL, int TP, int N, int CAP, int WG>
-__device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u32 r1, LeafLds<TP, N, CAP, WG>& s) {
+__device__ __forceinline__ u32 leaf_records(const SL& sl, const u32 r0, const u32 r1, LeafLds<TP, N, CAP, WG>& s) {
     u32 tid = threadIdx.x;
     pin(tid);  // addresses made from it are made again here, not kept in registers through the tile
     const u32 lane = tid & 63, wid = uniform(tid >> 6);
@@ -120,14 +121,17 @@ __device__ __forceinline__ void leaf_records(const SL& sl, const u32 r0, const u
         __syncthreads();
     }
     __syncthreads();
+    return tot;
 }
 
 // s.sum[i] = perft 2 of s.b[i] for i < np (np <= TP <= WG).  Every thread of
 // the workgroup calls it, with the boards stored (empty ones from np on to
 // the end of the last wave with parents) and a barrier behind them; it ends
-// with a barrier.
+// with a barrier.  `made` (when not null) grows by the parents' moves, summed
+// over the threads.
 template <class SL, int TP, int N, int CAP, int WG>
-__device__ __forceinline__ void leaf_tile(const SL& sl, const u32 np, LeafLds<TP, N, CAP, WG>& s) {
+__device__ __forceinline__ void leaf_tile(const SL& sl, const u32 np, LeafLds<TP, N, CAP, WG>& s,
+                                          u32* made = nullptr) {
     static_assert(TP == WG, "one parent per thread");
     static_assert(N >= 128, "one call of a whole wave fits");
     u32 tid = threadIdx.x;
@@ -140,11 +144,16 @@ __device__ __forceinline__ void leaf_tile(const SL& sl, const u32 np, LeafLds<TP
         e.nk = e.nf = e.call = 0;
         e.more = false;
         if (work) {
-            const u32 sum = leaf_sum(s.b[tid], sl, e);
-            if (!again) s.sum[tid] = sum;
+            u32 summed = 0;
+            const u32 sum = leaf_sum(s.b[tid], sl, e, made ? &summed : nullptr);
+            if (!again) {
+                s.sum[tid] = sum;
+                if (made) *made += summed;
+            }
         }
         if ((tid & 63) == 0) s.more[wid] = e.more;
-        leaf_records<false>(sl, N - e.nf, N, s);
+        const u32 full = leaf_records<false>(sl, N - e.nf, N, s);
+        if (made && tid == 0) *made += full;
         // (read between barriers, so that no wave writes the next round's yet)
         u32 m = 0;
 #pragma unroll

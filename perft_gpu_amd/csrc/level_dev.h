@@ -187,8 +187,11 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
                 const u32 e = s.mv[j];
                 const u32 par = (e >> 16) & (TP - 1);
                 const Board c = make_move(s.b[par], e & 0xFFFFu);
-                const u32 cc = count_moves(c, sl);
-                atomicAdd(&s.sum[par], cc);
+                u32 cc = 0;
+                if (!a.uncounted) {
+                    cc = count_moves(c, sl);
+                    atomicAdd(&s.sum[par], cc);
+                }
                 if (wr) {
                     a.out[base + j] = with_count(c, cc);
                     a.out_root[base + j] = s.root[par];

@@ -143,7 +143,8 @@ struct LdsEmitT {
     }
 };
 
-// The m children of one move-list window of a write level.  Every thread of
+// The m children of one move-list window of a write level (COUNT: with their
+// move counts).  Every thread of
 // the block calls it; it ends with the window's writes issued.
 // Two passes, so that the level's and the duplicate list's cursors -- one
 // address each, shared by every workgroup, whose atomics serialise -- move
@@ -153,7 +154,7 @@ struct LdsEmitT {
 //  2. one thread reserves both ranges; every child to be written or listed
 //     as a duplicate is made again with its keys and placed at a window-local
 //     cursor inside the reserved range.
-template <class SL>
+template <bool COUNT, class SL>
 __device__ __forceinline__ void write_window(const SL& sl, const TTArgs& a, const ZTables* zt, TTLds& s,
                                              const u32 p0, const u32 m, const int lane, const int wid) {
     const u64 below_mask = (1ULL << lane) - 1;
@@ -245,7 +246,7 @@ __device__ __forceinline__ void write_window(const SL& sl, const TTArgs& a, cons
                 if (keep) ck2 = zobrist_child(zt->k[1], s.k2[par], pb, mvv, black, c);
             }
         }
-        if (keep) {
+        if (COUNT && keep) {
             cc = count_moves(c, sl);
             atomicAdd(&s.sum[par], cc);
         }
@@ -279,7 +280,7 @@ __device__ __forceinline__ void write_window(const SL& sl, const TTArgs& a, cons
                 a.dup_slot[dpos] = (u32)probe_slot(ck1, a.dup_n, code >> 2);
             }
         }
-        if (a.out_bsum && nk) {
+        if (COUNT && a.out_bsum && nk) {
             // the wave's children are consecutive: at most two blocks
             const u64 b0 = first >> kBsumShift;
             const u64 part = keep ? (((pos >> kBsumShift) == b0) ? (u64)cc : (u64)cc << 32) : 0;
@@ -293,7 +294,7 @@ __device__ __forceinline__ void write_window(const SL& sl, const TTArgs& a, cons
 }
 
 // One tile (kTTP parents) of one level.  Every thread of the block calls it.
-template <class SL>
+template <bool COUNT = true, class SL>
 __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTables* zt, TTLds& s) {
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     {
@@ -354,7 +355,7 @@ __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTa
                     }
                 }
             } else {
-                write_window(sl, a, zt, s, p0, m, lane, wid);
+                write_window<COUNT>(sl, a, zt, s, p0, m, lane, wid);
             }
             __syncthreads();
         }
@@ -402,11 +403,11 @@ union TTAnyLds {
 // block calls it; it ends with a barrier.
 template <class SL>
 __device__ __forceinline__ void tt_leaf_sets(const SL& sl, const Board* in, unsigned long long* acc, const u32 np,
-                                             TTLeafLds& s) {
+                                             TTLeafLds& s, u32* made = nullptr) {
     const u32 tid = threadIdx.x;
     s.b[tid] = tid < np ? in[tid] : Board{};
     __syncthreads();
-    leaf_tile(sl, np, s);
+    leaf_tile(sl, np, s, made);
     if (tid < np) acc[tid] += s.sum[tid];
     __syncthreads();
 }
@@ -650,18 +651,21 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWav
 // after the other: 256 high-mobility positions at perft 6 71.3 -> 67.5 ms, one
 // middlegame position at perft 8 53.7 -> 51.3 ms.  The kept children of a tile are the windows'
 // reserved ranges (TTLds::wr_base/wr_n), whose accumulators the write just
-// zeroed; the leaf tiles add perft(child, 2) to them.
+// zeroed; the leaf tiles add perft(child, 2) to them, and their moves to the
+// level's total, so that the write need not count them (67.8 -> 66.0 ms).
 template <int B>
 __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_write_leaf(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
     __shared__ TTAnyLds s;
     __shared__ TTArgs sa;
     __shared__ u32 s_tile;
     __shared__ u32 s_nwin, s_base[kTTMaxWin], s_n[kTTMaxWin];
+    __shared__ unsigned long long s_made;
     const auto sl = SlOf<B>::make(tabs);
     const u32 total = t->tile_prefix[1];
     if (!t->fuse_leaf) return;  // the level was written by the write launch; the leaf launch follows
     if (blockIdx.x >= total) return;  // more workgroups than tiles: the others drain the queue
     copy_words(sa, t->seg[0]);
+    if (threadIdx.x == 0) s_made = 0;
     for (;;) {
         if (threadIdx.x == 0) s_tile = atomicAdd(&t->tile_ctr, 1u);
         __syncthreads();
@@ -670,7 +674,8 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWav
         {
             TTArgs a = uniform_args(sa);
             a.mode = kWrite;
-            tt_tile(sl, a, g, zt, s.w);  // ends with a barrier: the windows' ranges are final
+            a.total = nullptr;
+            tt_tile<false>(sl, a, g, zt, s.w);  // ends with a barrier: the windows' ranges are final
         }
         if (threadIdx.x < kTTMaxWin) {  // a leaf tile reuses the tile state
             s_base[threadIdx.x] = s.w.wr_base[threadIdx.x];
@@ -683,10 +688,15 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWav
             const u32 rb = __builtin_amdgcn_readfirstlane(s_base[w]), rn = __builtin_amdgcn_readfirstlane(s_n[w]);
             const Board* in = uniform_ptr(sa.out) + rb;
             unsigned long long* acc = uniform_ptr(sa.out_acc) + rb;
-            for (u32 c0 = 0; c0 < rn; c0 += kTTLeafParents)
-                tt_leaf_sets(sl, in + c0, acc + c0, min((u32)kTTLeafParents, rn - c0), s.l);
+            for (u32 c0 = 0; c0 < rn; c0 += kTTLeafParents) {
+                u32 made = 0;
+                tt_leaf_sets(sl, in + c0, acc + c0, min((u32)kTTLeafParents, rn - c0), s.l, &made);
+                made = wave_incl_scan(made);
+                if ((threadIdx.x & 63) == 63) atomicAdd(&s_made, (unsigned long long)made);
+            }
         }
     }
+    if (threadIdx.x == 0 && s_made) atomicAdd(sa.total, s_made);  // (behind the loop's last barrier)
 }
 
 // The serving step's write and leaf segments in one launch, overlapped:

@@ -46,11 +46,14 @@ u64 rnd() {
 extern "C" {
 
 // perft 2 by sets; stats: records, moves whose king replies were counted,
-// moves made and counted, records whose move number was wrong
+// moves made and counted, records whose move number was wrong (and 1 if the
+// moves summed and handed out are not all)
 uint64_t lc_perft2(const pf_pos48* p, int* stats) {
     const Board b = to_board(*p);
     Sum e{&b};
-    const uint64_t s = leaf_sum(b, sl, e);
+    u32 summed = 0;
+    const uint64_t s = leaf_sum(b, sl, e, &summed);
+    if (summed + (u32)e.full != count_moves(b, sl)) e.bad++;
     if (stats) stats[0] = e.recs, stats[1] = e.king, stats[2] = e.full, stats[3] = e.bad;
     return s + e.n;
 }

@@ -183,3 +183,25 @@ def test_serving_step_forms(pg, oracle, tt_bytes, jobs, n, dmax):
             assert got == {i: int(w) for i, w in want.items()}
     finally:
         eng.close()
+
+
+@pytest.mark.gpu
+def test_table_leaf_made_nodes(pg):
+    """the write level that runs with its leaf pass leaves its children's moves
+    to that pass: the same counts and the same number of children made as level
+    by level, where the write counts them"""
+    pos = pg.playouts(2024, 40, 15, 50, min_moves=35, no_check=True)
+    got = []
+    for graphs in (True, False):
+        eng = pg.Engine(arena_bytes=48 << 30, tt_bytes=1 << 30, zobrist_seed=3)
+        try:
+            eng.set_level_graphs(graphs)
+            eng.set_dedup(False)  # (which child claims a slot, and so which finds none, differs from run to run)
+            eng.reset_stats()
+            n = eng.perft_batch(pos, 6)
+            st = eng.stats()
+            got.append(([int(x) for x in n], st["made_nodes"], st["frontier_nodes"]))
+            assert (st["graph_passes"] > 0) == graphs
+        finally:
+            eng.close()
+    assert got[0] == got[1]
