@@ -552,8 +552,8 @@ def main():
     dout.free()
     leaves = int(counts.sum())
     value = leaves * args.steps / el
-    # per step: the root conversion, then the root count and depth - 1 level
-    # launches; gpu_ms holds the span from the root count to the last level
+    # per step: the begin kernel, depth - 1 level launches and the post kernel;
+    # gpu_ms holds the span from the begin kernel to the last level
     kernel_ms = st["gpu_ms"] / args.steps
     ops = W.C2_OPS_PER_LEAF * leaves
     achieved = ops / (kernel_ms * 1e-3) / 1e12
@@ -587,16 +587,16 @@ def main():
                      # HBM bytes per step: FETCH_SIZE x2.00 + WRITE_SIZE x1.00 over the step's kernels
                      # (rocprofv3 --pmc, calibrated on a copy of known size;
                      # profiles/k_stream_level_ks_c2_d5_counters.md)
-                     "traffic": 9.22e8,
+                     "traffic": 8.84e8,
                      "traffic_source": "profiles/k_stream_level_ks_c2_d5_counters.md (rocprofv3 --pmc "
                                        "FETCH_SIZE, WRITE_SIZE over one step, calibrated on a copy)",
-                     "kernel": ("k_stream_roots + %d x k_stream_level<%s>" % (depth - 1, args.backend)
+                     "kernel": ("k_stream_begin + %d x k_stream_write + k_stream_leaf<%s>" % (depth - 2, args.backend)
                                 if single == "stream" else "k_persistent<%s>" % args.backend),
                      "kernel_ms": kernel_ms,
                      "ops_per_leaf": W.C2_OPS_PER_LEAF,
                      # the hardware view: VALU wave-instructions issued per SIMD-cycle over the
                      # step (counted instructions per leaf, this run's kernel time, 1,024 SIMDs at
-                     # 2.4 GHz) against what the leaf loop's instruction mix can issue
+                     # 2.4 GHz) against what the leaf level's instruction mix can issue
                      "issue": issue_view(leaves, kernel_ms, args.backend)},
     }
 

@@ -38,7 +38,7 @@ struct Engine {
     u32 io_seq = 0;             // number of the last batch
     double clock_khz = 0;       // of the device clock in StreamIO
 
-    int grid[4][2] = {};        // level-loop launches on large levels (wide tile, five waves per SIMD)
+    int grid[4][2] = {};        // level-loop launches on large levels (write: wide tile; leaf: by sets)
     int grid_small[4][2] = {};  // the same on small levels (256 x 8192 tile)
     int pgrid[4] = {};
     int sgrid[4][2] = {};  // stream-ordered level launches: [backend][kLeaf / kWrite]

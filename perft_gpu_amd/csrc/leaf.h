@@ -8,7 +8,7 @@
 // children still made and 240 for each of the 3 whose king's replies are
 // counted: 9,800 in all.  Both are bound by the vector ALUs.  The leaf level
 // of 256 positions at perft 5 (8.16 million parents, 2.65e8 children): 4.79 ms
-// move by move, 1.99 ms by sets.  Most moves change only a few
+// move by move, 1.95 ms by sets.  Most moves change only a few
 // of the replies, and by an amount that the position itself tells: so the
 // replies are counted once, as if the opponent were to move in the position
 // (`base`), and a quiet move or capture from f to t changes that number by

@@ -221,13 +221,13 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
 // record pools hold ten records a parent and the move list 1,280 moves (a
 // tile of middlegame positions hands out some 820 records and 1,030 moves to
 // be counted in full, then 750 of which only the king's replies are), which
-// leaves room for three workgroups in a CU's LDS, as many as the kernel's 164
+// leaves room for three workgroups in a CU's LDS, as many as the kernel's 156
 // VGPRs allow.
 // Per-level kernels take it from kLeafSetsMinParents parents per workgroup: below,
 // a wave has too few parents for its long pass over each, and the leaf level
-// runs move by move.  16 roots at perft 4 (20 parents per workgroup): 60 us
-// move by move, 65 by sets; 32 roots (40): 86 against 83; 256 roots (320):
-// 283 against 179.
+// runs move by move.  16 roots at perft 4 (20 parents per workgroup): 54 us
+// either way; 32 roots (40): 86 move by move, 83 by sets; 256 roots (320): 283
+// against 179.
 constexpr int kLeafSetsWaves = 3;
 struct LeafLevelLds {
     LeafLds<256, 640, 1280, kWG> t;

@@ -19,7 +19,7 @@
 // run, and no cause in the source was found.  The leaf level's kernels are
 // kept free of spills for the same reason: built for four waves per SIMD (128
 // VGPRs, 44 B of spills per lane) their sums differed from run to run as soon
-// as two workgroups shared a compute unit, while the three-wave build (164
+// as two workgroups shared a compute unit, while the three-wave build (156
 // VGPRs, no spills) of the same source is exact and as fast.
 #include <hip/hip_runtime.h>
 
