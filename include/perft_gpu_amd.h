@@ -116,7 +116,8 @@ pf_status pf_pos_to_fen(const pf_pos48 *pos, char *buf, int buflen);
 
 /* perft(position, depth): replaces perftLauncher (launcher.h:1455-1504), which
  * prints instead of returning.  depth 0 -> 1.  Plain per-position path: a
- * host-driven level loop, no cross-position batching. */
+ * batch of one (without a table in stream order, and level by level from the
+ * host where a level does not fit the arena), no cross-position batching. */
 pf_status pf_perft(pf_ctx *ctx, const pf_pos48 *pos, int depth, uint64_t *out);
 
 /* Batched perft of n positions (any mix of sides to move): replaces
@@ -185,9 +186,9 @@ pf_status pf_set_tt_regions(pf_ctx *ctx, int log2_regions);
  * switches.h:14-21, and its launch-depth estimate, launcher.h:1535-1563): times
  * the current backend on `sample` (n positions, `depth`) over
  *   - the table-free single passes: the cooperative kernel's tile shapes and
- *     workgroups per CU, the stream-ordered level kernels' forms (tile shape x
- *     waves per SIMD, leaf and write level separately; for the byte-lookup
- *     backend also the form with its tables staged in LDS, form 6) and which
+ *     workgroups per CU, the stream-ordered write kernel's forms (tile shape x
+ *     waves per SIMD; for the byte-lookup backend also the form of both levels
+ *     with its tables staged in LDS, form 6) and which
  *     of the two passes PF_MODE_AUTO runs;
  *   - with a table: the level driver's write- and leaf-level workgroups per CU
  *     and, if the sample makes it chunk, the share of free memory a chunk's

@@ -69,6 +69,7 @@ pf_status Engine::init(const pf_config& cfg) {
     h_io->done = io_seq;
     int khz = 0;
     PF_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+    if (khz <= 0) return PF_EDEVICE;
     clock_khz = khz;
     PF_HIP(hipEventCreate(&ev0));
     PF_HIP(hipEventCreate(&ev1));
