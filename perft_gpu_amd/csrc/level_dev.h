@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "backends_dev.h"
+#include "gen_dev.h"
 #include "kernels.h"
 #include "leaf_dev.h"
 #include "wave.h"
@@ -75,6 +76,7 @@ struct TileLds {
     u32 wtot[WG / 64];
     unsigned long long red[WG / 64];
     u32 one[WG / 64];  // waves whose parents all have the tile's first root
+    u32 off[kCoopParents];
     u32 tile, base, ok;
 };
 static_assert(sizeof(TileLds<kByteLdsTP, kByteLdsCap, kByteLdsWG>) + kByteLds + 128 <= 160 * 1024,
@@ -154,6 +156,7 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
         }
         const u32 incl = wave_incl_scan(cnt);
         if (lane == 63) s.wtot[wid] = incl;
+        if (tid < (int)kCoopParents) s.off[tid] = incl - cnt;
         __syncthreads();
         u32 woff = 0, tot = 0;
 #pragma unroll
@@ -165,7 +168,9 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
         const u32 pre = woff + incl - cnt;
 
         for (u32 w0 = 0; w0 < tot; w0 += CAP) {
-            if (cnt && pre < w0 + CAP && pre + cnt > w0) {
+            if (WG == 256 && np <= kCoopParents) {
+                if constexpr (WG == 256) coop_generate<WG, CAP>(sl, s.b, s.off, np, s.mv);
+            } else if (cnt && pre < w0 + CAP && pre + cnt > w0) {
                 const Board b = s.b[tid];
                 PosInfo pi;
                 analyse(b, sl, pi);

@@ -334,37 +334,61 @@ PF_HD u32 count_pawns_knights(const Board& b, const PosInfo& pi, const CountMask
 
 // Legal move generation.  `emit(move)` is called once per legal move; the
 // order is: king, castles, knights, bishops, rooks, pawn pushes, double
-// pushes, captures, en passant.  Perft counts do not depend on it.
+// pushes, captures, en passant.  Perft counts do not depend on it.  Only the
+// pieces on the squares of `who` move.
+template <class Emit>
+PF_HD void emit_piece(Emit& emit, int s, u64 t) {  // from s to the squares of t
+    while (t) { emit(mk_move(s, ctz(t), kFlQuiet)); t &= t - 1; }
+}
+template <class Emit>
+PF_HD void emit_pawns(Emit& emit, int delta, u64 t) {  // from `delta` below the squares of t
+    while (t) {
+        const int d = ctz(t);
+        t &= t - 1;
+        if (d >= 56) {
+            emit(mk_move(d - delta, d, kFlPromoN)); emit(mk_move(d - delta, d, kFlPromoB));
+            emit(mk_move(d - delta, d, kFlPromoR)); emit(mk_move(d - delta, d, kFlPromoQ));
+        } else {
+            emit(mk_move(d - delta, d, kFlQuiet));
+        }
+    }
+}
+// Counts the moves instead.
+struct EmitCount {
+    u32 n;
+    PF_HD void operator()(u32) { n++; }
+};
+PF_HD void emit_piece(EmitCount& emit, int, u64 t) { emit.n = popc_add(t, emit.n); }
+PF_HD void emit_pawns(EmitCount& emit, int, u64 t) {
+    emit.n = popc_add(t, emit.n) + mul24((u32)popc(t & kRank8), 3);
+}
 template <class SL, class Emit>
-PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit) {
+PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit, u64 who = ~0ULL) {
     const u64 occ = pi.occ, us = pi.us, them = pi.them, empty = ~occ;
     const int ksq = pi.ksq;
-    const u64 P = pi.pawns & us, Pf = P & ~pi.pinned;
-    {
-        u64 t = king_fill(pi.K) & ~us & ~pi.att;
-        while (t) { emit(mk_move(ksq, ctz(t), kFlQuiet)); t &= t - 1; }
-    }
+    const u64 P = pi.pawns & us & who, Pf = P & ~pi.pinned;
+    const bool king = (pi.K & who) != 0;
+    if (king) emit_piece(emit, ksq, king_fill(pi.K) & ~us & ~pi.att);
     const bool check = pi.checkers != 0;
     if (check && (pi.checkers & (pi.checkers - 1))) return;
     const u64 tgt = check ? (pi.checkers | pi.block) : ~us;
     const u64 free = ~pi.pinned;
-    if (!check) {
+    if (king && !check) {
         const int r = st_rights(b);
         if ((r & 1) && !(occ & kF1G1) && !(pi.att & kF1G1)) emit(mk_move(4, 6, kFlOO));
         if ((r & 2) && !(occ & kB1D1) && !(pi.att & kC1D1)) emit(mk_move(4, 2, kFlOOO));
     }
     {
-        u64 N = b.knights & us & free;
+        u64 N = b.knights & us & free & who;
         while (N) {
             const int s = ctz(N);
             N &= N - 1;
-            u64 t = knight_fill(bit(s)) & tgt;
-            while (t) { emit(mk_move(s, ctz(t), kFlQuiet)); t &= t - 1; }
+            emit_piece(emit, s, knight_fill(bit(s)) & tgt);
         }
     }
     {
         const u64 kl[4] = {file_of(ksq), rank_of(ksq), diag_of(ksq), anti_of(ksq)};
-        u64 S = (b.bishops | b.rooks) & us;
+        u64 S = (b.bishops | b.rooks) & us & who;
         if (check) S &= free;
         while (S) {
             const int s = ctz(S);
@@ -375,7 +399,7 @@ PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit)
             if (b.rooks & sb) a |= sl.rook(s, occ);
             a &= tgt;
             if (pi.pinned & sb) a &= (kl[0] & sb) ? kl[0] : (kl[1] & sb) ? kl[1] : (kl[2] & sb) ? kl[2] : kl[3];
-            while (a) { emit(mk_move(s, ctz(a), kFlQuiet)); a &= a - 1; }
+            emit_piece(emit, s, a);
         }
     }
     {
@@ -385,33 +409,14 @@ PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit)
         const u64 Pnw = check ? Pf : (Pf | (P & pinA));
         const u64 p1 = (Ppush << 8) & empty;
         u64 t = p1 & tgt;
-        while (t) {
-            const int d = ctz(t);
-            t &= t - 1;
-            if (d >= 56) {
-                emit(mk_move(d - 8, d, kFlPromoN)); emit(mk_move(d - 8, d, kFlPromoB));
-                emit(mk_move(d - 8, d, kFlPromoR)); emit(mk_move(d - 8, d, kFlPromoQ));
-            } else {
-                emit(mk_move(d - 8, d, kFlQuiet));
-            }
-        }
+        emit_pawns(emit, 8, t);
         t = (((check ? (p1 & ~tgt) : p1) & kRank3) << 8) & empty & tgt;
         while (t) { const int d = ctz(t); t &= t - 1; emit(mk_move(d - 16, d, kFlDouble)); }
         for (int side = 0; side < 2; side++) {
             // a pawn pinned on a diagonal captures along it: its NE (a1-h8 pin) or
             // NW (a8-h1 pin) neighbour lies on the pin line by construction
-            u64 c = side ? (((Pnw << 7) & kNotH) & them & tgt) : (((Pne << 9) & kNotA) & them & tgt);
-            const int delta = side ? 7 : 9;
-            while (c) {
-                const int d = ctz(c);
-                c &= c - 1;
-                if (d >= 56) {
-                    emit(mk_move(d - delta, d, kFlPromoN)); emit(mk_move(d - delta, d, kFlPromoB));
-                    emit(mk_move(d - delta, d, kFlPromoR)); emit(mk_move(d - delta, d, kFlPromoQ));
-                } else {
-                    emit(mk_move(d - delta, d, kFlQuiet));
-                }
-            }
+            const u64 c = side ? (((Pnw << 7) & kNotH) & them & tgt) : (((Pne << 9) & kNotA) & them & tgt);
+            emit_pawns(emit, side ? 7 : 9, c);
         }
         const int ep = st_ep(b);
         if (ep) {

@@ -79,3 +79,20 @@ def test_contexts_on_threads(pg, oracle):
     for t in th:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("backend", ["ks", "plain", "fancy", "byte"])
+def test_parents_per_tile(pg, oracle, engine, backend):
+    """tiles of 4, 5, 8 and 9 parents (768 workgroups), whose moves are
+    generated by 64 and by 32 threads a parent and by one"""
+    pos = pg.playouts(21, 500, 2, 90)
+    want = oracle.perft_batch(pos, 2, nthreads=8)
+    engine.set_backend(backend)
+    try:
+        for n in (3071, 3072, 3073, 6143, 6144, 6145):
+            at = np.arange(n) % len(pos)
+            for mode in (pg.MODE_STREAM, pg.MODE_LEVELS):
+                got = engine.perft_batch(np.ascontiguousarray(pos[at]), 2, mode=mode)
+                assert np.array_equal(got, want[at]), (n, mode)
+    finally:
+        engine.set_backend("ks")
