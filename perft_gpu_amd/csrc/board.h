@@ -82,7 +82,15 @@ PF_HD u32 mul24(u32 a, u32 b) {
     return a * b;
 #endif
 }
-PF_HD int ctz(u64 x) { return __builtin_ctzll(x); }
+// (of 0, which only a side without a king asks for: 31, as the GPU's minimum of
+// the halves' find-first-bit results comes out)
+PF_HD int ctz(u64 x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_ctzll(x);
+#else
+    return x ? __builtin_ctzll(x) : 31;
+#endif
+}
 PF_HD u64 bit(int s) { return 1ULL << s; }
 PF_HD u64 flip(u64 x) { return __builtin_bswap64(x); }  // vertical mirror
 

@@ -536,7 +536,7 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit, u32* summed = nullp
                 ok = (T & ((kd & s) ? kd : (ka & s) ? ka : (kf & s) ? kf : rank_of(ksq))) != 0;
             } else if (s) {
                 const u64 pro = empty | C | s;
-                ok = !((att_e(b.rooks & them, pro) | att_w(b.rooks & them, pro)) & K);
+                ok = !((att_e(b.rooks & them, pro) | att_w(b.rooks & them, pro)) & K & kRank5);
             }
             emit(0, ok ? T : 0, (u32)(s ? ctz(s) : 0) | kLeafEP);
         }

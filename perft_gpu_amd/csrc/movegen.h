@@ -49,7 +49,7 @@ PF_HD u64 between_on(u64 line, int a, int b) {  // squares of `line` strictly be
 // for each sliding checker, the square just beyond the king on its line: the
 // one square that the threat map with our king removed (findAttackedSquares'
 // x-ray) adds to a map computed with the king in place, among the squares a
-// king move can reach.
+// king move can reach (and where we have several kings whatever it adds).
 PF_HD void pins_checks(const Board& b, PosInfo& pi, u64* xray) {
     const u64 pawns = b.pawns & kRanks2to7;
     const u64 occ = or3(or3(pawns, b.knights, b.bishops), b.rooks, b.kings);
@@ -76,6 +76,11 @@ PF_HD void pins_checks(const Board& b, PosInfo& pi, u64* xray) {
         } else if (!(in & (in - 1))) {
             pinned |= in & us;
         }
+    }
+    if (xray) {
+        // several kings of ours (a raw position may have them): the sliders' rays
+        // through all of them
+        if (__builtin_expect((K & (K - 1)) != 0, 0)) beyond = rook_fill(eR, ~(occ ^ K)) | bishop_fill(eB, ~(occ ^ K));
     }
     checkers |= and_or(knight_fill(K), eN, (((K << 7) & kNotH) | ((K << 9) & kNotA)) & eP);
     if (xray) *xray = beyond;
@@ -311,7 +316,7 @@ PF_HD u32 count_pawns_knights(const Board& b, const PosInfo& pi, const CountMask
                     const u64 s1 = ok & (0 - ok);
                     ok ^= s1;
                     const u64 pro = empty | C | s1;
-                    n += ((att_e(eR, pro) | att_w(eR, pro)) & pi.K) ? 0 : 1;
+                    n += ((att_e(eR, pro) | att_w(eR, pro)) & pi.K & kRank5) ? 0 : 1;
                 }
             } else {
                 n = popc_add(ok, n);
@@ -335,7 +340,8 @@ PF_HD u32 count_pawns_knights(const Board& b, const PosInfo& pi, const CountMask
 // Legal move generation.  `emit(move)` is called once per legal move; the
 // order is: king, castles, knights, bishops, rooks, pawn pushes, double
 // pushes, captures, en passant.  Perft counts do not depend on it.  Only the
-// pieces on the squares of `who` move.
+// pieces on the squares of `who` move; a side's king moves and castles belong
+// to its king's square, the lowest of several, and to a1 where it has none.
 template <class Emit>
 PF_HD void emit_piece(Emit& emit, int s, u64 t) {  // from s to the squares of t
     while (t) { emit(mk_move(s, ctz(t), kFlQuiet)); t &= t - 1; }
@@ -367,7 +373,7 @@ PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit,
     const u64 occ = pi.occ, us = pi.us, them = pi.them, empty = ~occ;
     const int ksq = pi.ksq;
     const u64 P = pi.pawns & us & who, Pf = P & ~pi.pinned;
-    const bool king = (pi.K & who) != 0;
+    const bool king = !~who || (who & (pi.K ? pi.K & (0 - pi.K) : 1));
     if (king) emit_piece(emit, ksq, king_fill(pi.K) & ~us & ~pi.att);
     const bool check = pi.checkers != 0;
     if (check && (pi.checkers & (pi.checkers - 1))) return;
@@ -434,7 +440,7 @@ PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit,
                     ok = (T & line) != 0;
                 } else {
                     const u64 pro = empty | C | s;
-                    ok = !((att_e(eR, pro) | att_w(eR, pro)) & pi.K);
+                    ok = !((att_e(eR, pro) | att_w(eR, pro)) & pi.K & kRank5);
                 }
                 if (ok) emit(mk_move(ctz(s), 40 + ep - 1, kFlEP));
             }
