@@ -44,8 +44,9 @@
 // replies of the opponent's king: it is summed without them and handed out as
 // a record of its own kind, for which only the king's moves and castling are
 // counted (leaf_king_replies).
-// A position in which the opponent is in check already, or a side has not
-// exactly one king, hands out every move.
+// A position in which the opponent is in check already, a side has not
+// exactly one king, or two pieces share a square (a castle with a right whose
+// rook is not at home may have put one on another piece) hands out every move.
 #pragma once
 #include "movegen.h"
 
@@ -300,7 +301,9 @@ PF_HD u32 leaf_sum(const Board& b, const SL& sl, Emit& emit, u32* summed = nullp
         thr = sc.thr;
         const u64 K = p.K;
         const u64 ours = or3(sc.att, knight_fill(b.knights & p.us), king_fill(K)) | pawn_hits(p.pawns & p.us);
-        generic = !eK || (eK & (eK - 1)) || !K || (K & (K - 1)) || (ours & eK);
+        const u64 pk = p.pawns | b.kings, sliders = b.bishops | b.rooks;
+        const u64 shared = or_and(or_and(p.pawns & b.kings, b.knights, sliders | pk), sliders, pk);
+        generic = !eK || (eK & (eK - 1)) || !K || (K & (K - 1)) || (ours & eK) || shared;
         // the opponent's king: moves, castling, and the squares both depend on
         u64 zone = king_fill(eK) & ~p.them;
         kings = popc_add(zone & ~ours, 0);

@@ -91,3 +91,40 @@ def test_levels_agree(pg, engine, backend):
             assert np.array_equal(engine.perft_batch(base, 2), got[0])
     finally:
         engine.set_backend("ks")
+
+
+def _bogus_rights(pg, seed, n):
+    """one king a side, back ranks thinned out, every castling right set: the
+    FEN parser takes rights whose king or rook is not at home, and a castle
+    then puts a rook where another piece may stand"""
+    pos = _random(pg, seed, n, 1, 1)
+    for name in pos.dtype.names:
+        if name not in ("kings", "white_pieces"):
+            pos[name] &= np.uint64(~0x7E0000000000007E & (1 << 64) - 1)
+    pos["pawns"] |= np.uint64(15)
+    return pos
+
+
+FENS = ["n6n/8/5P2/6K1/7R/2k5/5N2/8 b Qq - 0 1", "n4n2/5KRr/1bp3QP/3k3P/3p3p/3PQ2R/p2P3b/5Q2 b kq - 0 1",
+        "8/3k4/8/2K5/8/8/p6p/N6B w KQ - 0 1", "4k2n/8/8/8/8/8/5P2/4K2N b KQkq - 0 1"]
+
+
+def test_rights_without_rook(pg, kings):
+    pos = np.concatenate([pg.positions_array([pg.fen_to_pos(f) for f in FENS]), _bogus_rights(pg, 21, 600)])
+    bad = [(i, kings.kc_disagree(pos[i:].ctypes.data, 1)) for i in range(len(pos))]
+    bad = [x for x in bad if x[1]]
+    assert not bad, (len(bad), bad[:5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["ks", "plain", "fancy", "byte"])
+def test_rights_without_rook_levels(pg, engine, backend):
+    base = np.concatenate([pg.positions_array([pg.fen_to_pos(f) for f in FENS]), _bogus_rights(pg, 23, 60)])
+    engine.set_backend(backend)
+    try:
+        small = engine.perft_batch(base, 3)  # some 2,000 leaf parents: move by move
+        at = np.arange(4000) % len(base)
+        large = engine.perft_batch(np.ascontiguousarray(base[at]), 3)
+        assert np.array_equal(large, small[at])
+    finally:
+        engine.set_backend("ks")
