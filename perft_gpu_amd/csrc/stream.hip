@@ -14,13 +14,15 @@
 // perft_bb.h:327-329, switches.h:14-21).  The leaf level runs by sets (leaf.h).
 //
 // The write kernel's 256 x 4096 form built for five waves per SIMD (96
-// VGPRs, over 100 B of spills per lane) is not built: it gave counts that
-// differ from the oracle's on a perft 4 sample, and differently from run to
-// run, and no cause in the source was found.  The leaf level's kernels are
-// kept free of spills for the same reason: built for four waves per SIMD (128
-// VGPRs, 44 B of spills per lane) their sums differed from run to run as soon
-// as two workgroups shared a compute unit, while the three-wave build (156
-// VGPRs, no spills) of the same source is exact and as fast.
+// VGPRs, 20 to 32 B of spills per lane) is not built: an earlier state of it
+// gave counts on a perft 4 sample that differed from the oracle's and from run
+// to run, and no cause in the source was found.
+//
+// The leaf level's kernels are built for three waves per SIMD, the most that
+// needs no spills (tests/test_no_spills.py).  Built for four (128 VGPRs, 36 B
+// of spills per lane, record pools and move list cut so that four workgroups
+// fit a CU) 256 positions at perft 5 take 2.61 ms instead of 2.53, with equal
+// sums: 40 batches of all backends, eight runs each.
 #include <hip/hip_runtime.h>
 
 #include "convert.h"

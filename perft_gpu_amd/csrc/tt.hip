@@ -296,7 +296,9 @@ __device__ __forceinline__ void write_window(const SL& sl, const TTArgs& a, cons
 // One tile (kTTP parents) of one level.  Every thread of the block calls it.
 template <bool COUNT = true, class SL>
 __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTables* zt, TTLds& s) {
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    u32 id = threadIdx.x;
+    pin(id);  // what is made from it is made again for each tile, not kept in registers through a leaf tile
+    const int tid = (int)id, lane = tid & 63, wid = (int)uniform(id >> 6);
     {
         if (tid == 0) {
             s.nprobe = 0;
@@ -404,10 +406,12 @@ union TTAnyLds {
 template <class SL>
 __device__ __forceinline__ void tt_leaf_sets(const SL& sl, const Board* in, unsigned long long* acc, const u32 np,
                                              TTLeafLds& s, u32* made = nullptr) {
-    const u32 tid = threadIdx.x;
+    u32 tid = threadIdx.x;
+    pin(tid);  // (as in leaf_tile)
     s.b[tid] = tid < np ? in[tid] : Board{};
     __syncthreads();
     leaf_tile(sl, np, s, made);
+    pin(tid);
     if (tid < np) acc[tid] += s.sum[tid];
     __syncthreads();
 }
