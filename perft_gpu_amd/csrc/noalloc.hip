@@ -79,28 +79,34 @@ pf_status Engine::perft_noalloc(const pf_pos48* dpos, int n, int d, u64* dout) {
     p.arena_bytes = kScratchBytes - (ctl_b + roots_b + rid_b);
     p.ctl = ctl;
     p.sums = out;
+    // a launch that fails: what is queued reads the caller's positions and writes
+    // its counts, and has ended when the call returns
+    auto fail = [&] {
+        (void)hipStreamSynchronize(stream);
+        return PF_EDEVICE;
+    };
     const bool small = n <= (int)kStreamSmall && d >= 1;
     const int var[2] = {tune[backend].s_leaf, tune[backend].s_write};
     if (small) {
         if (launch_stream_small(backend, DevTables{d_tab}, p, dpos, sgrid[backend], var, stream) != hipSuccess)
-            return PF_EDEVICE;
+            return fail();
     } else {
         const u32 words = (u32)(sizeof(PersistCtl) / 4);
         const u32 clear_n = std::max<u32>((u32)n, words);
         hipLaunchKernelGGL(k_noalloc_clear, dim3((clear_n + 255) / 256), dim3(256), 0, stream, ctl, out, (u32)n,
                            d <= 0 ? 1ULL : 0ULL);
-        if (hipGetLastError() != hipSuccess) return PF_EDEVICE;
+        if (hipGetLastError() != hipSuccess) return fail();
         if (d <= 0) return hipStreamSynchronize(stream) == hipSuccess ? PF_OK : PF_EDEVICE;
-        if (launch_pos_to_board(dpos, (u32)n, roots, rid, stream) != hipSuccess) return PF_EDEVICE;
-        if (timing && hipEventRecord(ev0, stream) != hipSuccess) return PF_EDEVICE;
-        if (launch_stream(backend, DevTables{d_tab}, p, sgrid[backend], var, stream) != hipSuccess) return PF_EDEVICE;
-        if (timing && hipEventRecord(ev1, stream) != hipSuccess) return PF_EDEVICE;
+        if (launch_pos_to_board(dpos, (u32)n, roots, rid, stream) != hipSuccess) return fail();
+        if (timing && hipEventRecord(ev0, stream) != hipSuccess) return fail();
+        if (launch_stream(backend, DevTables{d_tab}, p, sgrid[backend], var, stream) != hipSuccess) return fail();
+        if (timing && hipEventRecord(ev1, stream) != hipSuccess) return fail();
     }
     st.kernel_launches += (u64)d + (small ? 1 : 3);  // the d - 1 levels and the kernels around them
     st.levels_run += (u64)(d - 1);
     // the overflow flag comes back through the host words allocated at init
     io_seq++;
-    if (launch_stream_post(p, out, d_io, io_seq, stream) != hipSuccess) return PF_EDEVICE;
+    if (launch_stream_post(p, out, d_io, io_seq, stream) != hipSuccess) return fail();
     const pf_status s2 = wait_small();
     // (the counts are complete for any stream or engine once the stream is)
     if (hipStreamSynchronize(stream) != hipSuccess) return PF_EDEVICE;
