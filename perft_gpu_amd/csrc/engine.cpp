@@ -319,6 +319,16 @@ void Engine::add_small_time() {
 // A batch of at most kStreamSmall roots (kernels.h).
 pf_status Engine::perft_stream_small(const pf_pos48* pos, int n, int d, u64* out, bool dev_in, bool dev_out) {
     PF_HIP(hipSetDevice(device));
+    if (dev_out) {
+        // the post kernel writes `out` itself: a buffer too small for the counts
+        // is refused here, as the runtime's copy of a larger batch refuses it
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipMemGetAddressRange(&base, &size, out) != hipSuccess)
+            (void)hipGetLastError();
+        else if (reinterpret_cast<char*>(out) + (size_t)n * 8 > static_cast<char*>(base) + size)
+            return PF_EDEVICE;
+    }
     pf_status s = ensure_sums((u64)n);
     if (s != PF_OK) return s;
     char* mark = arena + arena_top;
