@@ -199,13 +199,7 @@ pf_status pf_perft(pf_ctx* ctx, const pf_pos48* pos, int depth, uint64_t* out) {
     if (!ctx || !pos || !out || check_depth(depth)) return PF_EINVAL;
     std::lock_guard<std::recursive_mutex> g(ctx->eng.mu);
     if (ctx->eng.serving) return PF_EBUSY;
-    // the stream-ordered pass (no table: one wait instead of one per level);
-    // the level driver where a table is used or a level does not fit
-    if (!(ctx->eng.d_tt && depth >= 3)) {
-        const pf_status s = ctx->eng.perft_stream(pos, 1, depth, out);
-        if (s != PF_ENOMEM) return s;
-    }
-    return ctx->eng.perft_levels(pos, 1, depth, out);
+    return ctx->eng.perft_one(pos, depth, out);
 }
 
 // Where a caller's buffer lives: 0 host (pageable, pinned or managed), 1 device

@@ -362,9 +362,25 @@ pf_status Engine::perft_stream_small(const pf_pos48* pos, int n, int d, u64* out
     if (s != PF_OK) return s;
     // device results: complete for any stream or engine once the stream is
     if (dev_out && hipStreamSynchronize(stream) != hipSuccess) return PF_EDEVICE;
+    st.peak_arena_bytes = std::max<u64>(st.peak_arena_bytes, (u64)(p.arena - arena) + h_io->used);
     add_small_time();
     if (!dev_out) memcpy(out, h_io->sums, (size_t)n * 8);
     return PF_OK;
+}
+
+// One position: the stream-ordered pass (one wait instead of one per level);
+// the level driver where a table is used or a level does not fit (after the
+// levels that do: 1 to 9% of such a call).
+pf_status Engine::perft_one(const pf_pos48* pos, int d, u64* out) {
+    if (!(d_tt && d >= 3)) {
+        const pf_status s = perft_stream(pos, 1, d, out);
+        if (s == PF_OK && d >= 1 && timing) {  // per level, as the level driver reports them
+            st.last_expand_launches = (u64)(d - 1);
+            st.last_expand_ms = d > 1 ? st.last_expand_ms / (d - 1) : 0.0;
+        }
+        if (s != PF_ENOMEM) return s;
+    }
+    return perft_levels(pos, 1, d, out);
 }
 
 pf_status Engine::perft_stream(const pf_pos48* pos, int n, int d, u64* out, bool dev_in, bool dev_out) {

@@ -108,6 +108,7 @@ struct Engine {
     void destroy();
     pf_status ensure_sums(u64 n);
     pf_status perft_levels(const pf_pos48* pos, int n, int depth, u64* out);
+    pf_status perft_one(const pf_pos48* pos, int depth, u64* out);
     // dev_in / dev_out: `pos` / `out` are device memory of this engine's device
     pf_status perft_persistent(const pf_pos48* pos, int n, int depth, u64* out, bool dev_in = false,
                                bool dev_out = false);

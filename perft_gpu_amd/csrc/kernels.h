@@ -115,6 +115,7 @@ struct StreamIO {  // coherent host memory
     u32 done;      // the call's number, written after the rest
     u32 err;       // PersistCtl::err
     unsigned long long t0, t1;  // device clock at the begin and the post kernel
+    unsigned long long used;    // arena bytes of the levels written
     unsigned long long sums[kStreamSmall];
     pf_pos48 pos[kStreamSmall];
 };

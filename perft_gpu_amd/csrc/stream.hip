@@ -85,11 +85,21 @@ __global__ __launch_bounds__(kStreamSmall) void k_stream_begin(const SliderTable
     }
 }
 
-__global__ __launch_bounds__(kWG) void k_stream_post(const PersistCtl* ctl, const unsigned long long* sums, u32 n,
-                                                     unsigned long long* out, StreamIO* io, u32 seq) {
+// Arena bytes of a level of n nodes: its boards, then its root ids.
+__device__ __forceinline__ u64 level_bytes(u64 n) {
+    return ((n * sizeof(Board) + 255) & ~255ULL) + ((n * sizeof(u32) + 255) & ~255ULL);
+}
+
+__global__ __launch_bounds__(kWG) void k_stream_post(const PersistCtl* ctl, int depth, const unsigned long long* sums,
+                                                     u32 n, unsigned long long* out, StreamIO* io, u32 seq) {
     if (threadIdx.x == 0) {
-        io->err = ctl->err;
-        io->t0 = ctl->t0;
+        const int L = depth > 2 ? depth - 2 : 0;  // the last level written, behind the roots
+        // (all read before the first is written)
+        const u32 err = ctl->err;
+        const unsigned long long t0 = ctl->t0, off = ctl->lvl_off[L], nodes = ctl->totals[L];
+        io->err = err;
+        io->t0 = t0;
+        io->used = L ? off + level_bytes(nodes) : 0;
         io->t1 = wall_clock64();
     }
     for (u32 i = threadIdx.x; i < n; i += blockDim.x) out[i] = sums[i];
@@ -122,7 +132,7 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
         off = lo;
         cur = reinterpret_cast<const Board*>(p.arena + off);
         cur_r = reinterpret_cast<const u32*>(p.arena + off + ((n * sizeof(Board) + 255) & ~255ULL));
-        off += ((n * sizeof(Board) + 255) & ~255ULL) + ((n * sizeof(u32) + 255) & ~255ULL);
+        off += level_bytes(n);
     }
     LevelArgs a;
     a.in = cur;
@@ -296,7 +306,7 @@ hipError_t launch_stream_small(int backend, const DevTables& dt, const PersistAr
 hipError_t launch_stream_post(const PersistArgs& a, unsigned long long* dev_out, StreamIO* io, u32 seq, hipStream_t s) {
     const u32 n = dev_out == a.sums ? 0u : a.n_roots;  // counts to move
     if (!dev_out && n > kStreamSmall) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_stream_post, dim3(1), dim3(n > 64 ? kWG : 64), 0, s, a.ctl, a.sums, n,
+    hipLaunchKernelGGL(k_stream_post, dim3(1), dim3(n > 64 ? kWG : 64), 0, s, a.ctl, a.depth, a.sums, n,
                        dev_out ? dev_out : io->sums, io, seq);
     return hipGetLastError();
 }
