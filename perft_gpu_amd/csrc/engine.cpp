@@ -67,10 +67,9 @@ pf_status Engine::init(const pf_config& cfg) {
     PF_HIP(hipHostMalloc(&h_io, sizeof(StreamIO), hipHostMallocCoherent | hipHostMallocMapped));
     PF_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&d_io), h_io, 0));
     h_io->done = io_seq;
-    int khz = 0;
-    PF_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
-    if (khz <= 0) return PF_EDEVICE;
-    clock_khz = khz;
+    int khz = 0;  // (a device that does not tell: small batches are timed by events)
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess) (void)hipGetLastError();
+    clock_khz = khz > 0 ? khz : 0;
     PF_HIP(hipEventCreate(&ev0));
     PF_HIP(hipEventCreate(&ev1));
     PF_HIP(hipMalloc(&d_pctl, sizeof(PersistCtl)));
@@ -310,7 +309,14 @@ pf_status Engine::wait_small() {
 
 void Engine::add_small_time() {
     if (!timing) return;
-    const double ms = (double)(h_io->t1 - h_io->t0) / clock_khz;
+    double ms = 0;
+    if (time_by_events()) {
+        float f = 0;
+        if (hipEventSynchronize(ev1) != hipSuccess || hipEventElapsedTime(&f, ev0, ev1) != hipSuccess) return;
+        ms = f;
+    } else {
+        ms = (double)(h_io->t1 - h_io->t0) / clock_khz;
+    }
     st.gpu_ms += ms;
     st.last_expand_ms = ms;
     st.last_expand_launches = 1;
@@ -349,8 +355,10 @@ pf_status Engine::perft_stream_small(const pf_pos48* pos, int n, int d, u64* out
     if (!dev_in) memcpy(h_io->pos, pos, (size_t)n * sizeof(pf_pos48));
     const int var[2] = {tune[backend].s_leaf, tune[backend].s_write};
     io_seq++;
-    if (launch_stream_small(backend, DevTables{d_tab}, p, dev_in ? pos : d_io->pos, sgrid[backend], var, stream) !=
+    if ((time_by_events() && hipEventRecord(ev0, stream) != hipSuccess) ||
+        launch_stream_small(backend, DevTables{d_tab}, p, dev_in ? pos : d_io->pos, sgrid[backend], var, stream) !=
             hipSuccess ||
+        (time_by_events() && hipEventRecord(ev1, stream) != hipSuccess) ||
         launch_stream_post(p, dev_out ? reinterpret_cast<unsigned long long*>(out) : nullptr, d_io, io_seq, stream) !=
             hipSuccess) {
         (void)hipStreamSynchronize(stream);  // what was launched may still read the positions

@@ -36,7 +36,7 @@ struct Engine {
     StreamIO* h_io = nullptr;   // small stream-ordered batches: positions in, outcome back
     StreamIO* d_io = nullptr;   // h_io as the device addresses it
     u32 io_seq = 0;             // number of the last batch
-    double clock_khz = 0;       // of the device clock in StreamIO
+    double clock_khz = 0;       // of the device clock in StreamIO (0: not known)
 
     int grid[4][2] = {};        // level-loop launches on large levels (write: wide tile; leaf: by sets)
     int grid_small[4][2] = {};  // the same on small levels (256 x 8192 tile)
@@ -135,6 +135,7 @@ struct Engine {
     pf_status range_count(const Board* b, u64 n, u64* total);
     // Waits for the batch that launch_stream_post posts as io_seq; adds its time.
     pf_status wait_small();
+    bool time_by_events() const { return timing && !(clock_khz > 0); }
     void add_small_time();
     pf_status perft_stream_small(const pf_pos48* pos, int n, int depth, u64* out, bool dev_in, bool dev_out);
     pf_status upload_roots(const pf_pos48* pos, int n, Board** roots, u32** rid, bool dev_in = false);

@@ -88,8 +88,10 @@ pf_status Engine::perft_noalloc(const pf_pos48* dpos, int n, int d, u64* dout) {
     const bool small = n <= (int)kStreamSmall && d >= 1;
     const int var[2] = {tune[backend].s_leaf, tune[backend].s_write};
     if (small) {
+        if (time_by_events() && hipEventRecord(ev0, stream) != hipSuccess) return fail();
         if (launch_stream_small(backend, DevTables{d_tab}, p, dpos, sgrid[backend], var, stream) != hipSuccess)
             return fail();
+        if (time_by_events() && hipEventRecord(ev1, stream) != hipSuccess) return fail();
     } else {
         const u32 words = (u32)(sizeof(PersistCtl) / 4);
         const u32 clear_n = std::max<u32>((u32)n, words);
