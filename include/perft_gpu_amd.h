@@ -186,9 +186,9 @@ pf_status pf_set_tt_regions(pf_ctx *ctx, int log2_regions);
  * switches.h:14-21, and its launch-depth estimate, launcher.h:1535-1563): times
  * the current backend on `sample` (n positions, `depth`) over
  *   - the table-free single passes: the cooperative kernel's tile shapes and
- *     workgroups per CU, the stream-ordered write kernel's forms (tile shape x
- *     waves per SIMD; for the byte-lookup backend also the form of both levels
- *     with its tables staged in LDS, form 6) and which
+ *     workgroups per CU, the stream-ordered write kernel's tile shapes (for
+ *     the byte-lookup backend also the form of both levels with its tables
+ *     staged in LDS, form 6) and which
  *     of the two passes PF_MODE_AUTO runs;
  *   - with a table: the level driver's write- and leaf-level workgroups per CU
  *     and, if the sample makes it chunk, the share of free memory a chunk's

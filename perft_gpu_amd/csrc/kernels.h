@@ -90,13 +90,14 @@ hipError_t launch_persistent(int backend, int variant, const DevTables& dt, cons
 // The same batch as one launch per level on stream s (levels sized and placed
 // on the device; no host round trip): the root count, then depth - 1 level
 // launches of grid[kWrite] / grid[kLeaf] workgroups of the level kernel's
-// form variant[kWrite] / variant[kLeaf].  Write levels have kStreamWriteVariants
-// forms (stream.hip: tile shape * 3 + waves per SIMD target), the leaf level
-// one, by sets; both have one more for the byte backend.
-constexpr int kStreamWriteVariants = 5;  // (there is no five-wave 256 x 4096 write form)
+// form variant[kWrite] / variant[kLeaf].  Write levels have two forms, the leaf
+// level one, by sets; both have one more for the byte backend.  (The numbers
+// are those of tune files.)
+constexpr int kStreamWrite8192 = 0;      // 256 parents x 8192 moves a tile
+constexpr int kStreamWrite4096 = 3;      // 256 x 4096
 constexpr int kStreamByteLds = 6;        // byte backend only: its tables staged in LDS (both modes)
 constexpr int kStreamLeafSets = 7;       // leaf level by sets (leaf.h); below kLeafSetsMinParents move by move
-constexpr int kStreamWriteDefault = 3;   // 256 x 4096 tile, no waves target
+constexpr int kStreamWriteDefault = kStreamWrite4096;
 int stream_grid(int backend, int mode, int variant, int n_cu);
 hipError_t launch_stream(int backend, const DevTables& dt, const PersistArgs& a, const int grid[2],
                          const int variant[2], hipStream_t s);

@@ -8,15 +8,13 @@
 // Every workgroup of a level launch derives the same placement from words
 // the previous launch finished writing.
 //
-// The write kernel is built in kStreamWriteVariants forms -- two tile shapes
-// times three waves-per-SIMD targets, less the last -- of which the autotuner
-// picks one per backend (the reference fixes its launch shape at compile time,
-// perft_bb.h:327-329, switches.h:14-21).  The leaf level runs by sets (leaf.h).
-//
-// The write kernel's 256 x 4096 form built for five waves per SIMD (96
-// VGPRs, 20 to 32 B of spills per lane) is not built: an earlier state of it
-// gave counts on a perft 4 sample that differed from the oracle's and from run
-// to run, and no cause in the source was found.
+// The write kernel is built in two forms, a move window of 8192 and one of
+// 4096, of which the autotuner picks one per backend (the reference fixes its
+// launch shape at compile time, perft_bb.h:327-329, switches.h:14-21).  Their
+// LDS and registers (124 VGPRs) hold them at three and four workgroups per CU;
+// asked for four or five waves per SIMD the first compiles to the same
+// instructions, the second for four too, and for five (96 VGPRs) it spills.
+// The leaf level runs by sets (leaf.h).
 //
 // The leaf level's kernels are built for three waves per SIMD, the most that
 // needs no spills (tests/test_no_spills.py).  Built for four (128 VGPRs, 36 B
@@ -29,18 +27,6 @@
 #include "level_dev.h"
 
 namespace pf {
-
-// Variant v = shape * 3 + waves: shape 0 is the 256 x 8192 tile (PCfg
-// variant 0), shape 1 the 256 x 4096 tile (PCfg variant 2); waves 0, 1, 2 ask
-// the compiler for no target, four and five resident waves per SIMD.
-template <int SH>
-struct StreamShape {
-    static constexpr int v = SH ? 2 : 0;
-};
-template <int WV>
-struct StreamWaves {
-    static constexpr int v = WV == 2 ? 5 : WV == 1 ? 4 : 1;
-};
 
 template <int B>
 __global__ __launch_bounds__(kWG) void k_stream_roots(const SliderTables* tabs, PersistArgs p) {
@@ -187,10 +173,9 @@ __device__ __forceinline__ void stream_level(const MakeSl& make_sl, const Persis
     expand_level(sl, a, kWrite, s);
 }
 
-template <int B, int SH, int WV>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(StreamWaves<WV>::v)))
-void k_stream_write(const SliderTables* tabs, PersistArgs p, int L) {
-    using Shape = PCfg<B, StreamShape<SH>::v>;
+template <int B, int V>
+__global__ __launch_bounds__(kWG) void k_stream_write(const SliderTables* tabs, PersistArgs p, int L) {
+    using Shape = PCfg<B, V>;
     __shared__ TileLds<Shape::TP, Shape::CAP, kWG> s;
     stream_level<kWrite, false>([&] { return SlOf<B>::make(tabs); }, p, L, s, nullptr);
 }
@@ -220,13 +205,8 @@ void k_stream_leaf(const SliderTables* tabs, PersistArgs p, int L) {
 template <int B>
 static void* level_fn(int mode, int v) {
     if (mode == kLeaf) return reinterpret_cast<void*>(&k_stream_leaf<B>);
-    switch (v) {
-    case 0: return reinterpret_cast<void*>(&k_stream_write<B, 0, 0>);
-    case 1: return reinterpret_cast<void*>(&k_stream_write<B, 0, 1>);
-    case 2: return reinterpret_cast<void*>(&k_stream_write<B, 0, 2>);
-    case 3: return reinterpret_cast<void*>(&k_stream_write<B, 1, 0>);
-    default: return reinterpret_cast<void*>(&k_stream_write<B, 1, 1>);
-    }
+    return v == kStreamWrite8192 ? reinterpret_cast<void*>(&k_stream_write<B, 0>)
+                                 : reinterpret_cast<void*>(&k_stream_write<B, 2>);
 }
 static void* pick_stream_level(int backend, int mode, int v) {
     if (backend == kByte && v == kStreamByteLds)

@@ -34,8 +34,11 @@ void Engine::apply_tuning() {
         // (files may name leaf forms 0 to 5, which ran every leaf move by move
         // and are no longer built)
         if (!(lds_form_ok && t.s_leaf == kStreamByteLds)) t.s_leaf = kStreamLeafSets;
-        if (t.s_write < 0 || (t.s_write >= kStreamWriteVariants && !(lds_form_ok && t.s_write == kStreamByteLds)))
-            t.s_write = kStreamWriteDefault;
+        // (files may name write forms 1, 2 and 4, waves-per-SIMD targets that made
+        // no difference to forms 0 and 3)
+        if (t.s_write == 1 || t.s_write == 2) t.s_write = kStreamWrite8192;
+        if (t.s_write != kStreamWrite8192 && !(lds_form_ok && t.s_write == kStreamByteLds))
+            t.s_write = kStreamWrite4096;
         if (t.tt_chunk_pct < 10 || t.tt_chunk_pct > 90) t.tt_chunk_pct = 50;
         const int pmax = persistent_max_bpc(b, t.p_variant);
         const int pb = (t.p_bpc > 0 && t.p_bpc < pmax) ? t.p_bpc : pmax;
@@ -129,8 +132,8 @@ pf_status Engine::save_tuning(const char* path) const {
 //  kTuneSinglePass: every tile shape x workgroups-per-CU of the cooperative
 //    kernel, then the stream-ordered form against the best of them, with the
 //    byte backend's two leaf-level forms and, with the best of these, the
-//    write-level kernel's forms (tile shape x waves per SIMD); kernel
-//    time from HIP events, best of three after a warm-up.
+//    write-level kernel's forms; kernel
+//    time from HIP events or the device clock, best of three after a warm-up.
 //  kTuneTable (with a table): the level driver's write-level and leaf-level
 //    workgroups per CU and, when the sample makes the driver chunk, the share
 //    of the free arena a chunk's next level may take; whole-call time, best
@@ -194,9 +197,10 @@ pf_status Engine::autotune(const pf_pos48* pos, int n, int d, int what) {
             double stream_ms = 1e30;
             for (int pass = 0; pass < 2 && s == PF_OK; pass++) {
                 // the forms of this mode, and for the byte backend its LDS form
-                const int forms = pass == 0 ? 1 : kStreamWriteVariants, nsv = forms + (b == kByte ? 1 : 0);
-                for (int i = 0; i < nsv; i++) {
-                    const int v = i >= forms ? kStreamByteLds : pass == 0 ? kStreamLeafSets : i;
+                std::vector<int> forms = {kStreamLeafSets};
+                if (pass == 1) forms = {kStreamWrite8192, kStreamWrite4096};
+                if (b == kByte) forms.push_back(kStreamByteLds);
+                for (const int v : forms) {
                     if (pass == 0) tune[b].s_leaf = v; else tune[b].s_write = v;
                     apply_tuning();
                     double ms = 0;
