@@ -80,7 +80,7 @@ PF_HD void pins_checks(const Board& b, PosInfo& pi, u64* xray) {
     if (xray) {
         // several kings of ours (a raw position may have them): the sliders' rays
         // through all of them
-        if (__builtin_expect((K & (K - 1)) != 0, 0)) beyond = rook_fill(eR, ~(occ ^ K)) | bishop_fill(eB, ~(occ ^ K));
+        if (K & (K - 1)) beyond = rook_fill(eR, ~(occ ^ K)) | bishop_fill(eB, ~(occ ^ K));
     }
     checkers |= and_or(knight_fill(K), eN, (((K << 7) & kNotH) | ((K << 9) & kNotA)) & eP);
     if (xray) *xray = beyond;
@@ -341,7 +341,7 @@ PF_HD u32 count_pawns_knights(const Board& b, const PosInfo& pi, const CountMask
 // order is: king, castles, knights, bishops, rooks, pawn pushes, double
 // pushes, captures, en passant.  Perft counts do not depend on it.  Only the
 // pieces on the squares of `who` move; a side's king moves and castles belong
-// to its king's square, the lowest of several, and to a1 where it has none.
+// to its king's square, the lowest of several, and to ctz(0) where it has none.
 template <class Emit>
 PF_HD void emit_piece(Emit& emit, int s, u64 t) {  // from s to the squares of t
     while (t) { emit(mk_move(s, ctz(t), kFlQuiet)); t &= t - 1; }
@@ -373,7 +373,7 @@ PF_HD void generate(const Board& b, const SL& sl, const PosInfo& pi, Emit& emit,
     const u64 occ = pi.occ, us = pi.us, them = pi.them, empty = ~occ;
     const int ksq = pi.ksq;
     const u64 P = pi.pawns & us & who, Pf = P & ~pi.pinned;
-    const bool king = !~who || (who & (pi.K ? pi.K & (0 - pi.K) : 1));
+    const bool king = !~who || ((who >> ksq) & 1);
     if (king) emit_piece(emit, ksq, king_fill(pi.K) & ~us & ~pi.att);
     const bool check = pi.checkers != 0;
     if (check && (pi.checkers & (pi.checkers - 1))) return;
