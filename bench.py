@@ -14,11 +14,15 @@ persistent cooperative launch (grid barriers between levels) and through the
 host-driven level loop under "backends".
 
 Also reported on the same box, outside the timed region:
-  roofline      integer-VALU roofline of the step's kernels: algorithmic int32
-                lane-ops per step (C2 op model x leaves) / the step's kernel
-                time (HIP events on the engine's stream around the level
-                launches) against MI355X's published vector rate,
-                157.3 TFLOP/s FP32 = 78.6 T lane-op/s
+  roofline      integer-VALU roofline of the step's kernels: the lane-
+                instructions they issue per step (counted, per leaf) / the
+                step's kernel time (device clock, from its first kernel to its
+                last level) against MI355X's published vector rate, 157.3
+                TFLOP/s FP32 = 78.6 T lane-op/s; issue: the same against what
+                their instruction mix can issue; op_model: the reference
+                algorithm's lane-ops (C2 op model x leaves) in that time,
+                which is no fraction of a roof, as the leaf sums answer them
+                with a fifth of the instructions
   plain         the same 256 positions through the plain per-position path
   backends      batched nodes/sec per slider backend, and the level modes
   serving       C4: the whole configured stream (Poisson arrivals, 50 req/s
@@ -555,8 +559,10 @@ def main():
     # per step: the begin kernel, depth - 1 level launches and the post kernel;
     # gpu_ms holds the span from the begin kernel to the last level
     kernel_ms = st["gpu_ms"] / args.steps
-    ops = W.C2_OPS_PER_LEAF * leaves
-    achieved = ops / (kernel_ms * 1e-3) / 1e12
+    # (instructions per leaf are counted for the Kogge-Stone kernels)
+    counted = W.C2_VALU_LANE_INSTR_PER_LEAF if args.backend == "ks" and single == "stream" else None
+    achieved = counted * leaves / (kernel_ms * 1e-3) / 1e12 if counted else None
+    model = W.C2_OPS_PER_LEAF * leaves / (kernel_ms * 1e-3) / 1e12
     log("timed: %.3f s, %.3e nodes/s, kernel %.3f ms" % (el, value, kernel_ms))
 
     line = {
@@ -583,7 +589,7 @@ def main():
                                   "one persistent cooperative launch",
                    "tuning": tuning},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_TOPS, "unit": "Tlane-op/s",
-                     "frac": achieved / VALU_PEAK_TOPS,
+                     "frac": achieved / VALU_PEAK_TOPS if achieved else None,
                      # HBM bytes per step: FETCH_SIZE x2.00 + WRITE_SIZE x1.00 over the step's kernels
                      # (rocprofv3 --pmc, calibrated on a copy of known size;
                      # profiles/k_stream_level_ks_c2_d5_counters.md)
@@ -593,7 +599,8 @@ def main():
                      "kernel": ("k_stream_begin + %d x k_stream_write + k_stream_leaf<%s>" % (depth - 2, args.backend)
                                 if single == "stream" else "k_persistent<%s>" % args.backend),
                      "kernel_ms": kernel_ms,
-                     "ops_per_leaf": W.C2_OPS_PER_LEAF,
+                     "op_model": {"ops_per_leaf": W.C2_OPS_PER_LEAF, "rate": model,
+                                  "over_peak": model / VALU_PEAK_TOPS},
                      # the hardware view: VALU wave-instructions issued per SIMD-cycle over the
                      # step (counted instructions per leaf, this run's kernel time, 1,024 SIMDs at
                      # 2.4 GHz) against what the leaf level's instruction mix can issue

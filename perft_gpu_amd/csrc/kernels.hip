@@ -12,7 +12,8 @@
 //          kLeaf : add the count to the parent's LDS sum (depth-1 nodes), or
 //          kWrite: also append the child (count in its Board) to the next level
 //     -> per-root sums: one 64-bit atomic per tile when the tile has a single
-//        root (the common case), else one per parent; plus the level total.
+//        root (the common case), else one per run of parents with the same
+//        root in each wave; plus the level total.
 //
 // The LDS move list replaces the reference's global move array, its scan and
 // its interval-expand (the parent index rides in the list entry), and the

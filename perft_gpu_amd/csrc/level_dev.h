@@ -226,7 +226,7 @@ __device__ __forceinline__ void expand_level(const SL& sl, const LevelArgs& a, c
 // record pools hold ten records a parent and the move list 1,280 moves (a
 // tile of middlegame positions hands out some 820 records and 1,030 moves to
 // be counted in full, then 750 of which only the king's replies are), which
-// leaves room for three workgroups in a CU's LDS, as many as the kernel's 156
+// leaves room for three workgroups in a CU's LDS, as many as the kernel's 158
 // VGPRs allow.
 // Per-level kernels take it from kLeafSetsMinParents parents per workgroup: below,
 // a wave has too few parents for its long pass over each, and the leaf level

@@ -111,7 +111,7 @@ class Server {
     u32* h_rb_ = nullptr;          // pinned staging of block-sum read-backs (rb_cap_ entries)
     u64 rb_cap_ = 0;
     u32 late_src_[kMaxLate] = {};  // their write segments (indices before the reordering)
-    // by tiling (1: fine), late leaf launch (1: recorded), then upsweep rounds
+    // by form of the step, late leaf launch (1: recorded), then upsweep rounds
     hipGraph_t graph_[kStepForms][2][kUpRounds + 1] = {};
     hipGraphExec_t exec_[kStepForms][2][kUpRounds + 1] = {};
     u64 steps_ = 0, segs_ = 0, dups_ = 0;

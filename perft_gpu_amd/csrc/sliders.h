@@ -5,13 +5,19 @@
 //          tables.  Counting uses one fill per direction over ALL movers of
 //          that direction at once: rays of different pieces in one direction
 //          never overlap, so popcount(fill & targets) is the exact move count.
+//          A single slider's attacks are two lines by obstruction difference.
 //   Plain  per-square magics, private 4096/512-entry windows, 2.25 MiB
 //          (MoveGeneratorBitboard.h:810-827; magics found by a seeded search).
 //   Fancy  fixed-shift fancy magics sharing one 97,264-entry table, 760 KiB
 //          (MoveGeneratorBitboard.h:753-790; published constants).
 //   Byte   the same magics indexing a u8 table of per-square unique-attack
-//          slots, 146 KiB in total (MoveGeneratorBitboard.h:762-770); on the
-//          GPU every workgroup stages it in LDS.
+//          slots, 146 KiB in total (MoveGeneratorBitboard.h:762-770), read
+//          through the caches or, in one form of the stream-ordered kernels,
+//          from a copy in LDS.
+//
+// The backend decides how moves are generated and made children counted.  The
+// leaf level's sums (leaf.h) fill the lines of both sides' sliders whatever the
+// backend and ask it for our single sliders' attacks only.
 //
 // Every backend returns attacks including the first blocker in each direction;
 // callers mask own pieces.

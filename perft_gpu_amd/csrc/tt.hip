@@ -393,8 +393,8 @@ __device__ void tt_tile(const SL& sl, const TTArgs& a, const u32 tile, const ZTa
 // workgroup.  One workgroup's LDS holds either a table tile or a leaf tile.
 // The leaf children are not made and counted one by one (841 vector
 // instructions each) but summed by sets: 256 high-mobility positions at perft 6
-// 117.9 -> 68.6 ms, one middlegame position at perft 8 91 -> 61 ms, a burst of
-// 200 requests 40.3 -> 31.4 ms, same results.
+// 117.5 -> 64.8 ms, one middlegame position at perft 8 74.7 -> 50.8 ms, a burst
+// of 200 requests 52.0 -> 42.8 ms, same results.
 using TTLeafLds = LeafLds<kTTLeafParents, 640, 1280, kTWG>;
 union TTAnyLds {
     TTLds w;
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWav
 // segment's children; their number is that write's outcome (none if it
 // overflowed), so the tile prefix is built here, by the first wave.
 template <int B>
-__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_late(const SliderTables* tabs, const ZTables* zt, StepTable* t) {
+__global__ __launch_bounds__(kTWG) __attribute__((amdgpu_waves_per_eu(kTTLeafWaves))) void k_step_late(const SliderTables* tabs, StepTable* t) {
     __shared__ TTAnyLds s;
     __shared__ u32 pre[kMaxLate + 1], s_n[kMaxLate];
     __shared__ const Board* s_in[kMaxLate];
@@ -1125,8 +1125,10 @@ int step_grid(int backend, int n_cu) {
 // cover kMaxRoots and kMaxSegs (the roots and the outcomes are handled by the
 // first threads of the start kernel).  A small step's fetch and start are one
 // launch, and so are its upsweeps and outcomes, as each of its kernels is a
-// launch's latency (4 to 5 us) and little else: a request at depth 4 on an idle
-// server, two steps, 95.8 -> 89.2 us.
+// launch's latency (4 to 5 us) and little else.  A request at depth 4 on an idle
+// server, two steps: 91.6 us with leaf passes move by move, 95.7 with the larger
+// kernels of those by sets, 92.6 with a first tile by index, 89.2 with fewer
+// launches.
 template <int B, bool F>
 static void launch_step_front(const SliderTables* tabs, const ZTables* zt, StepTable* t, const StepTable* h, uint4* tt,
                               u64 mask, int grid, int up_grid, bool small, int late, hipStream_t s) {
@@ -1137,7 +1139,7 @@ static void launch_step_front(const SliderTables* tabs, const ZTables* zt, StepT
         hipLaunchKernelGGL(k_pre_step<B>, dim3(up_grid), dim3(256), 0, s, tabs, t, t->seg, tt, mask);
     }
     hipLaunchKernelGGL((k_step_mixed<B, F>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
-    if (late) hipLaunchKernelGGL((k_step_late<B>), dim3(grid), dim3(kTWG), 0, s, tabs, zt, t);
+    if (late) hipLaunchKernelGGL((k_step_late<B>), dim3(grid), dim3(kTWG), 0, s, tabs, t);
 }
 
 hipError_t launch_step(int backend, const SliderTables* tabs, const ZTables* zt, StepTable* t, StepTable* h, uint4* tt,

@@ -158,7 +158,8 @@ struct StepTable {
     // the write tiles, the others on the leaf tiles
     u32 mix_write_wgs;
     // parents per tile of the mixed launch's finely tiled form (its tile
-    // prefix counts with it); the other form tiles by kTTTileParents
+    // prefix counts with it); the coarse form tiles write segments by
+    // kTTTileParents and leaf segments by kTTLeafParents
     u32 mix_tp;
     // planned pass: the last write level runs its leaf pass fused (set by its
     // planner when the level has enough tiles for every workgroup)
@@ -256,8 +257,8 @@ int step_max_bpc(int backend, int leaf);  // the planned pass's write (0) / leaf
 // once every outcome is visible to the host.
 // late: the late leaf launch is recorded (steps with StepTable::nlate > 0).
 enum StepForm {
-    kStepCoarse,  // the mixed launch tiles by kTTTileParents parents
-    kStepFine,    // ... by StepTable::mix_tp
+    kStepCoarse,  // the mixed launch tiles by kTTTileParents parents, leaf segments by kTTLeafParents
+    kStepFine,    // ... both by StepTable::mix_tp
     kStepSmall,   // fine, within the kSmall* bounds: fewer launches
     kStepForms
 };

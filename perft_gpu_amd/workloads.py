@@ -98,12 +98,14 @@ C2_LEAVES = 8988346871
 C2_MADE_NODES = 8001 + 249956 + 8164767 + 265225172
 C2_OPS_PER_MADE_NODE = 416777397783 / C2_MADE_NODES
 # What the hardware issues for the same step with the Kogge-Stone kernels
-# (rocprofv3 --pmc SQ_INSTS_VALU on one C2 step: 1.2447e9 wave-instructions in
-# the leaf level, 3.0799e7 in the three write levels), per leaf, as lane-
+# (rocprofv3 --pmc SQ_INSTS_VALU on one C2 step: 1.249e9 wave-instructions in
+# the leaf level, 3.456e7 in the three write levels), per leaf, as lane-
 # instructions; and the most wave-instructions per SIMD-cycle the leaf level's
-# instruction mix can issue: 3,597 of the 5,808 VALU instructions of its path
-# by sets issue every ~2.4 cycles (two-input logic, bitop3, add, moves), 2,211
-# every ~4.2 (shifts, popcounts, selects, compares, perms), measured per opcode
-# with all waves resident, i.e. 5,808 instructions per 17,919 cycles.
-C2_VALU_LANE_INSTR_PER_LEAF = (1.2447e9 + 3.0799e7) * 64 / 8988346871
-C2_LOOP_ISSUE_LIMIT = 5808 / 17919
+# instruction mix can issue.  Two-input logic, bitop3, add and moves issue every
+# ~2.4 cycles; shifts, popcounts, selects, compares and perms every ~4.2
+# (measured per opcode with all waves resident).  The fast share is 63% in the
+# sums, 62% in the children made, 58% in the king replies and 42% in the
+# records' lists, of which 64 parents issue about 4,900, 3,480, 720 and 690
+# instructions: 9,790 in 30,360 cycles.
+C2_VALU_LANE_INSTR_PER_LEAF = (1.249e9 + 3.456e7) * 64 / 8988346871
+C2_LOOP_ISSUE_LIMIT = 9790 / 30360
