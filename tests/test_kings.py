@@ -128,3 +128,27 @@ def test_rights_without_rook_levels(pg, engine, backend):
         assert np.array_equal(large, small[at])
     finally:
         engine.set_backend("ks")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["ks", "fancy"])
+def test_serving_several_kings(pg, engine, backend):
+    """the serving thread sizes a request's levels with the host's own count"""
+    pos = np.concatenate([_random(pg, 9, 30, w, b) for w, b in ((2, 2), (3, 1), (1, 0), (None, None))])
+    engine.set_backend(backend)
+    try:
+        want = engine.perft_batch(pos, 3)
+    finally:
+        engine.set_backend("ks")
+    eng = pg.Engine(backend=backend, arena_bytes=1 << 30)
+    try:
+        eng.serve_start(max_jobs=32)
+        for i in range(len(pos)):
+            eng.submit(pos[i], 3, i)
+        got = {}
+        while len(got) < len(pos):
+            got.update((r["tag"], (r["status"], r["nodes"])) for r in eng.poll())
+        eng.serve_stop()
+        assert got == {i: (0, int(w)) for i, w in enumerate(want)}
+    finally:
+        eng.close()
