@@ -137,8 +137,13 @@ pf_status Server::build_graph(StepForm form, int late, int rounds) {
         if (g) hipGraphDestroy(g);
         return PF_EDEVICE;
     }
+    hipGraphExec_t x = nullptr;
+    if (hipGraphInstantiate(&x, g, nullptr, nullptr, 0) != hipSuccess) {
+        hipGraphDestroy(g);  // (a later step tries again)
+        return PF_EDEVICE;
+    }
     graph_[form][late][rounds] = g;
-    if (hipGraphInstantiate(&exec_[form][late][rounds], g, nullptr, nullptr, 0) != hipSuccess) return PF_EDEVICE;
+    exec_[form][late][rounds] = x;
     return PF_OK;
 }
 
